@@ -70,11 +70,15 @@ int q8_0_set_tune(const char *key, int value);  // "q8_0_gemv.rows" / ".depth"
 #define DOE_Q4K_BLOCK_ELEMS 256
 
 // gelu_tanh with the reference's clamp of the tanh argument
-// (gelu_gated.wgsl:5-8, reference_interpreter.zig:1027-1045).
+// (gelu_gated.wgsl:5-8, reference_interpreter.zig:1027-1045): 0.5 x (1 +
+// tanh u) written as x / (1 + e^-2u), which keeps its relative accuracy where
+// 1 + tanh u cancels, in one exp2 and one reciprocal; below -9.02 the f32
+// tanh is -1 and the factor 0.
 __device__ __forceinline__ float doe_gelu_tanh_clamped(float x) {
     float inner = 0.7978845608028654f * (x + 0.044715f * x * x * x);
     inner = fminf(fmaxf(inner, -15.0f), 15.0f);
-    return 0.5f * x * (1.0f + tanhf(inner));
+    const float f = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(inner * -2.8853900817779268f));
+    return x * (inner < -9.02f ? 0.0f : f);
 }
 
 __device__ __forceinline__ float doe_half_bits_to_float(uint32_t bits16) {
