@@ -113,6 +113,40 @@ def test_q8_0_gemm_f32(dev, ora, m, n, k):
     assert rel_l2(got[0], y0) <= EXACT_TOL
 
 
+@pytest.mark.parametrize("fmt", ["q4k", "q8_0"])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (31, 127, 31), (33, 129, 257), (64, 128, 320), (65, 130, 511),
+                                   (129, 640, 1100), (200, 9000, 512)])
+def test_gemm_f32_tile_edges(dev, ora, fmt, m, n, k):
+    # around the edges of the 32-row fragments, the 64 / 128 x 128 tiles and
+    # the 32 / 64 / 256 pieces of K, without and with K splits, plain, with the
+    # residual and with GeGLU of column pairs.  Bound: A's two f16 parts carry
+    # it to 2^-22, f32 sums of k terms to 2^-24 sqrt(k), the minima's sums
+    # cancel against the scales' (a factor of 2).
+    from doe_amd import q8_0
+
+    rng = np.random.default_rng(m + 3 * n + k)
+    a = (rng.standard_normal((m, k)) * 10.0 ** rng.uniform(-3, 3, (m, 1))).astype(np.float32)
+    w = q4k.random_q4k(rng, n, k) if fmt == "q4k" else q8_0.random_q8_0(rng, n, k)
+    wf = (ora.q4k_dequant_rowwise if fmt == "q4k" else ora.q8_0_dequant)(w, n, k).astype(np.float64)
+    want = a.astype(np.float64) @ wf.T
+    tol = 2 * (2.0 ** -22 + 2.0 ** -24 * np.sqrt(k))
+    da, dw = up(a), up(w)
+    out = DeviceBuffer.empty((m, n), np.float32)
+    ops.matmul_gemm_f32_fused(da, dw, out, m, n, k, fmt)
+    got = out.download()
+    for r in range(m):  # every row on its own scale
+        assert rel_l2(got[r], want[r]) <= tol, r
+    res = (rng.standard_normal((m, n)) * np.abs(want).max(1, keepdims=True)).astype(np.float32)
+    x = up(res)
+    ops.matmul_gemm_f32_fused(da, dw, x, m, n, k, fmt, residual=x)
+    assert np.array_equal(x.download(), got + res)
+    if n % 2 == 0:
+        h, hw = DeviceBuffer.empty((m, n // 2), np.float32), DeviceBuffer.empty((m, n // 2), np.float32)
+        ops.matmul_gemm_f32_fused(da, dw, h, m, n, k, fmt, activation=ops.GEGLU_PAIRS)
+        ops.geglu_pairs(out, hw, m * (n // 2))
+        assert np.array_equal(h.download(), hw.download())
+
+
 def test_gemm_prefill_config_sampled(dev, ora):
     # the 31B-class prefill shape: M=2048 tokens, K=5376, N=21504; the oracle
     # evaluates 2048 sampled entries (every row once, at a random column)
