@@ -191,3 +191,40 @@ def test_prefill_f16kv_decoder_layout(dev, ora, hq, hkv, d, mq_splits):
     err = rel_l2(got, want)
     print(f"[mq decoder layout {hq}/{hkv}x{d} splits {mq_splits}] rel_l2 {err:.2e}", flush=True)
     assert err <= 1e-3, err
+
+
+@pytest.mark.parametrize("d,hq,hkv,ql,start,maxs,window,layout", [
+    (64, 4, 2, 2, 0, 40, 0, 0), (64, 2, 2, 33, 97, 140, 0, 1), (64, 8, 1, 300, 0, 300, 50, 0),
+    (128, 4, 4, 31, 1, 64, 0, 0), (128, 6, 3, 65, 300, 400, 128, 1), (128, 2, 1, 17, 3000, 3100, 0, 0),
+    (256, 4, 2, 32, 0, 32, 0, 1), (256, 8, 4, 129, 31, 200, 33, 0), (256, 2, 1, 5, 2043, 2100, 0, 0),
+    (256, 1, 1, 96, 0, 96, 1, 0)])
+def test_prompt_blocks_against_float64(dev, d, hq, hkv, ql, start, maxs, window, layout):
+    # around the edges of the 32-query and 32-key blocks, fewer blocks than
+    # waves, windows that skip blocks, long caches (keys split over the grid);
+    # cache rows past the prompt hold NaN (never written).  Bound: scores of
+    # |s| < 8 from two f16 parts of Q (2^-22), P in two f16 parts (2^-22), f32
+    # sums over kv keys (2^-24 sqrt(kv)).
+    rng = np.random.default_rng(d + ql + start)
+    kv = start + ql
+    q = (rng.standard_normal((ql, hq, d)) * 10.0 ** rng.uniform(-2, 0.3, (ql, hq, 1))).astype(np.float32)
+    k = np.full((hkv, maxs, d), np.nan, np.float16)
+    v = np.full((hkv, maxs, d), np.nan, np.float16)
+    k[:, :kv] = rng.standard_normal((hkv, kv, d))
+    v[:, :kv] = rng.standard_normal((hkv, kv, d))
+    scale = 1.0 / np.sqrt(d)
+    out = DeviceBuffer.empty((ql, hq, d), np.float32)
+    order = (0, 1, 2) if layout == 0 else (1, 0, 2)
+    ops.attention_prefill_f16kv(up(q), up(k.transpose(order)), up(v.transpose(order)), out, num_heads=hq,
+                                num_kv_heads=hkv, head_dim=d, query_len=ql, kv_len=kv, kv_stride=maxs,
+                                start_pos=start, scale=scale, sliding_window=window, kv_layout=layout)
+    got = out.download().astype(np.float64)
+    pos, key = np.arange(start, kv)[:, None], np.arange(kv)[None, :]
+    seen = (key <= pos) & ((key > pos - window) if window else True)
+    for h in range(hq):
+        g = h // (hq // hkv)
+        s = q[:, h].astype(np.float64) @ k[g, :kv].astype(np.float64).T * scale
+        s = np.where(seen, s, -np.inf)
+        p = np.exp(s - s.max(1, keepdims=True))
+        want = p @ v[g, :kv].astype(np.float64) / p.sum(1, keepdims=True)
+        tol = 2.0 ** -22 * (8 + 1) + 2.0 ** -24 * np.sqrt(kv)
+        assert rel_l2(got[:, h], want) <= tol, (h, rel_l2(got[:, h], want))
