@@ -7,9 +7,11 @@
 // [q_len][Hq][128], k/v bf16 [Hkv][kv_stride][128] (the cache layout
 // [kv_head][pos][dim]), out f32 or bf16 [q_len][Hq][128].
 //
-// One workgroup = 128 queries of one head (four waves of 32), keys in blocks
-// of 64 staged in LDS (double-buffered, the next block's loads in flight).
-// Per wave and key block:
+// One workgroup = four or eight waves: 64 or 128 rows (32 or 64 queries of two
+// heads that share K and V, of one head where the group is odd), each 32 of
+// them to two waves that take one half of the keys each.  Keys are staged in LDS
+// in blocks of 64, K by direct loads, V through registers as f16.
+// Per wave and key block (32 keys of it):
 //   * S^T = K . Q^T on v_mfma_f32_32x32x16_bf16 (bf16 inputs are exact, f32
 //     accumulate).  The transposed product puts one query per lane column, so
 //     the online softmax needs no cross-lane reductions except one exchange
@@ -17,23 +19,31 @@
 //   * P = exp2(S*scale*log2e - m) in f32 (one fma and one exp per score),
 //     rounded to f16, and O^T += V^T . P^T on v_mfma_f32_32x32x16_f16: P's
 //     registers are used in place as the B operand (the key order of the
-//     product follows the MFMA's D layout; V^T is read in the same order).
-//     The row sum l adds the same f16 P values (v_dot2_f32_f16).
+//     product follows the MFMA's D layout; V is read transposed in the same
+//     order).  The row sum l adds the same f16 P values (v_dot2_f32_f16).
 //   * The running max m is raised (and O, l rescaled) only when some query's
 //     block max exceeds it by more than 2^8: P stays <= 256, well inside f16,
 //     and the O rescale runs on a few blocks instead of every block.
 //   * The causal mask is evaluated only on the blocks that cross the
 //     diagonal (or the end of the keys); blocks every query sees fully skip it.
-// V is converted once per call by a pre-pass into an f16 V^T copy [Hkv][128]
-// [keys] (exact for |v| in [2^-14, 65504]; f16 P keeps the output near 1e-4
-// rel-L2, where a bf16 P would sit at ~1e-3), so the main loop copies V^T
-// tiles straight into LDS.
-// Query blocks are dispatched heavy and light in complementary halves so the
-// two workgroups resident on a CU carry about the same number of key blocks.
+// V in f16 is exact for |v| in [2^-14, 65504]; f16 P keeps the output near 1e-4
+// rel-L2, where a bf16 P would sit at ~1e-3.  The two key halves merge their (O,
+// m, l) through LDS at the end.
+//
+// What bounds it: at 2048 queries x 32 / 16 heads, all CUs full, the clock (1.8
+// GHz under this load, 2.3 with half of the CUs at work; 2130 cycles per block
+// and wave pair in both, of which the matrix cores take 1024 and the vector
+// unit about 1300); otherwise the workgroup with the most key blocks.  us, with
+// 128 queries of one head per workgroup, every wave reading all keys (32 KB of
+// LDS per 32 MFMAs, the LDS port's own rate) and V^T from a pre-pass, in
+// brackets: 2048 x 32 / 16 heads 47.8 (54.6); 2048 x 8 / 8 26.8 (44.6); 1500
+// after 512 x 4 / 4 24.3 (43.0); 1100 x 32 / 16 23.1 (34.8); 65 x 4 / 4 6.2
+// (10.6).  Two tiles of 32 rows to a wave (half of the LDS reads, one wave per
+// SIMD) took 55 and 43 on the first two; three blocks of K in flight instead of
+// two, or a block's first K operands read before the barrier, changed nothing.
 #include "common.h"
 
 #include <math.h>
-#include <mutex>
 
 namespace {
 
@@ -42,26 +52,29 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kD = 128, kBQ = 128, kBKV = 64;
-constexpr int kKRow = kD + 8;    // bf16 per K row in LDS (272 B: b128 reads conflict-free)
-constexpr int kVRow = kBKV + 4;  // f16 per V^T row in LDS (136 B = 34 dwords: 16 lanes' b64 reads hit 32 distinct banks)
-constexpr float kLazy = 8.0f;    // the running max is raised only past m + 8 (P <= 2^8)
+constexpr int kD = 128, kBKV = 64;
+constexpr float kLazy = 8.0f;  // the running max is raised only past m + 8 (P <= 2^8)
+constexpr int kBlock = kBKV * kD * 2;  // bytes of a staged K or V block
+constexpr int kKRing = 3, kVRing = 2;
+constexpr int kLds = (kKRing + kVRing) * kBlock;
+static_assert(8 * 64 * (128 + 8) <= kLds, "the merge's state (eight waves' 64 lanes x 32 floats, m and l) fits the rings");
 
 struct PrefillArgs {
-    const uint16_t *q, *k;
-    const _Float16 *vt;  // f16 V^T [hkv][kD][kv_pad], keys >= kv_len zero
+    const uint16_t *q, *k, *v;
     void *out;
-    int hq, hkv, q_len, kv_len, kv_stride, kv_pad, start_pos, causal, out_bf16, nqb;
+    int hq, hkv, q_len, kv_len, kv_stride, start_pos, causal, out_bf16;
+    int pair, units, cols;  // heads of a workgroup's tiles 2 c, 2 c + 1 (pair) or c; query units; c's count
     float scale_log2;  // softmax scale * log2(e)
 };
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float float2v __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ uint32_t bf16pair_to_f16pair(uint32_t w) {
-    const float lo = __uint_as_float(w << 16), hi = __uint_as_float(w & 0xffff0000u);
-    const _Float16 a = (_Float16)lo, b = (_Float16)hi;
-    return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+    const float2v f = {__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u)};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, half2v));
 }
 
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
@@ -70,317 +83,323 @@ __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
     return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
 
-// Pre-pass: V bf16 [hkv][kv_stride][128] -> f16 V^T [hkv][128][kv_pad] (keys
-// past kv_len zero); one workgroup per 64 keys of one KV head, transposed
-// through LDS.
-__global__ __launch_bounds__(256) void v_to_f16t_kernel(const uint16_t *__restrict__ v, _Float16 *__restrict__ vt,
-                                                        int kv_len, int kv_stride, int kv_pad) {
-    __shared__ _Float16 tile[kBKV][kD + 2];  // [key][dim], odd dword stride
-    const int kvh = blockIdx.y, key0 = blockIdx.x * kBKV, tid = threadIdx.x;
-    // the four loads go out together (a key past kv_len reads a clamped key
-    // and is zeroed after: no branch, so no load waits for the one before)
-    u32x4 wl[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int gi = tid + 256 * i, kl = gi >> 4, d0 = (gi & 15) * 8;
-        const int key = max(min(key0 + kl, kv_len - 1), 0);
-        wl[i] = *reinterpret_cast<const u32x4 *>(v + ((size_t)kvh * kv_stride + key) * kD + d0);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int gi = tid + 256 * i, kl = gi >> 4, d0 = (gi & 15) * 8;
-        const uint32_t keep = key0 + kl < kv_len ? 0xffffffffu : 0u;  // (an and: the load is used either way)
-        const u32x4 w = wl[i] & keep;
-        const uint32_t p[4] = {bf16pair_to_f16pair(w.x), bf16pair_to_f16pair(w.y), bf16pair_to_f16pair(w.z),
-                               bf16pair_to_f16pair(w.w)};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t *>(&tile[kl][d0 + 2 * e]) = p[e];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int gi = tid + 256 * i, d = gi >> 3, k0 = (gi & 7) * 8;
-        half8 r;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) r[j] = tile[k0 + j][d];
-        *reinterpret_cast<half8 *>(vt + ((size_t)kvh * kD + d) * kv_pad + key0 + k0) = r;
-    }
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t rsrc, void *lds, uint32_t lane_off, uint32_t off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)lds, 16, lane_off, off, 0, 0);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(PrefillArgs a) {
-    __shared__ __attribute__((aligned(16))) uint16_t Ks[2][kBKV * kKRow];
-    __shared__ __attribute__((aligned(16))) _Float16 Vt[2][kD * kVRow];
+// A transposed read of LDS.  (As the access of a restrict parameter: without
+// alias information the compiler holds it back until every load to LDS has landed.)
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+__device__ __forceinline__ s16x4 read_tr(lds_s16x4 *__restrict__ p) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16(p); }
 
-    const int h = blockIdx.x % a.hq;
-    const int slot = blockIdx.x / a.hq;
-    const int half = (a.nqb + 1) / 2;
-    const int qb = slot < half ? a.nqb - 1 - slot : slot - half;
-    const int kvh = h / (a.hq / a.hkv);
-    const int q0 = qb * kBQ;
+// max / sum over the two lane halves that hold the same query
+__device__ __forceinline__ float halves_max(float x) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+}
+__device__ __forceinline__ float halves_sum(float x) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+}
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// At most N vector-memory operations outstanding, no LDS operation, and every
+// wave here: what they wrote to LDS can be read.  (Not a fence: that would wait
+// for the loads to LDS that are still under way.)
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (0 << 8) | (((N >> 4) & 3) << 14));
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+}
+
+template <int W>
+__global__ __launch_bounds__(64 * W, 8 / W) void attn_prefill_kernel(PrefillArgs a) {
+    constexpr int kExchange = W * 64 * 128;  // the merge: the waves' 64 lanes x 32 floats
+    constexpr int NP = 16 / W, kStep = kBlock / NP;  // 16-byte loads of a thread per staged block
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 31, lg = lane >> 5;
-    const int qi = q0 + wave * 32 + lr;  // this lane's query (column of S^T)
-    const int qrow = min(qi, a.q_len - 1);
+    const int qt = wave % (W / 2), kh = wave / (W / 2);
+    // the units of the last queries see the most keys: first
+    const int col = blockIdx.x % a.cols, unit = a.units - 1 - blockIdx.x / a.cols;
+    const int uq = a.pair ? 8 * W : 16 * W;  // queries of a unit
+    const int q0 = unit * uq, q_end = min(q0 + uq, a.q_len);
+    const int head = a.pair ? 2 * col + (qt & 1) : col, kvh = head / (a.hq / a.hkv);
+    const int kv_end = a.causal ? min(a.kv_len, a.start_pos + q_end) : a.kv_len;
+    const int nkb = (kv_end + kBKV - 1) / kBKV;
+    // this lane's query (column of S^T) and the keys [0, limit) that it sees
+    const int qi = q0 + 32 * (a.pair ? qt >> 1 : qt) + lr;
+    const int limit = qi < a.q_len && a.causal ? min(a.kv_len, a.start_pos + qi + 1) : kv_end;
 
     // Q^T operand fragments: Q[qi][h][16 s + 8 lg .. + 8]
     bf16x8 qf[8];
     {
-        const uint16_t *qp = a.q + ((size_t)qrow * a.hq + h) * kD + 8 * lg;
+        const uint16_t *qp = a.q + ((size_t)min(qi, a.q_len - 1) * a.hq + head) * kD + 8 * lg;
 #pragma unroll
         for (int s = 0; s < 8; ++s) qf[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(qp + 16 * s));
     }
 
-    const int q_last = min(q0 + kBQ, a.q_len) - 1;
-    const int kv_end = a.causal ? min(a.kv_len, a.start_pos + q_last + 1) : a.kv_len;
-    const int nkb = (kv_end + kBKV - 1) / kBKV;
-    // keys this lane's query may see: [0, limit)
-    const int limit = qi < a.q_len ? (a.causal ? min(a.kv_len, a.start_pos + qi + 1) : a.kv_len) : kv_end;
-
-    // K and V^T of this KV head as buffers: per-lane offsets fixed for the whole
-    // loop, the block offset a scalar; keys past kv_len read as zero (masked)
+    // K and V of this KV head as buffers: per-lane offsets fixed for the whole
+    // loop, the block a scalar; keys past kv_len read as zero (masked).  A row
+    // of 16 chunks; place c' of row `key` holds chunk c' ^ (key & 15) of K, c' ^
+    // 4 (key & 3) of V, so that the lanes' reads fall on different banks.
     const __amdgpu_buffer_rsrc_t krsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(a.k + (size_t)kvh * a.kv_stride * kD), (short)0, a.kv_len * (kD * 2), 0x00020000);
     const __amdgpu_buffer_rsrc_t vrsrc = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(a.vt + (size_t)kvh * kD * a.kv_pad), (short)0, a.kv_pad * (kD * 2), 0x00020000);
-    // K staging: granule gi = tid + 256 i -> key gi >> 4, column (gi & 15) * 8
-    // V^T staging: dim tid >> 1, keys 32 (tid & 1) + 8 i .. + 7 of the block
-    const int vd = tid >> 1, vh = tid & 1;
-    const uint32_t k_voff = (uint32_t)((tid >> 4) * kD + (tid & 15) * 8) * 2u;  // + 16 keys per i
-    const uint32_t v_voff = (uint32_t)(vd * a.kv_pad + 32 * vh) * 2u;           // + 8 keys per i
-    // K runs one block ahead of V: in iteration kb, Ks[(kb + 1) & 1] holds
-    // K(kb + 1) (the next block's scores are computed under this block's
-    // softmax) and Vt[kb & 1] holds V(kb); K(kb + 2) and V(kb + 1) are loaded
-    // during the iteration and written to the buffers freed by the previous
-    // iteration's barrier.  Out-of-range block indices are clamped: their
-    // loads stay inside the buffers and their results are never used.
-    u32x4 rk[4], rv[4];
-#define DOE_PF_LOAD_K(KB)                                                                            \
-    _Pragma("unroll") for (int i = 0; i < 4; ++i) rk[i] = __builtin_amdgcn_raw_buffer_load_b128(     \
-        krsrc, k_voff + (uint32_t)i * (16 * kD * 2), (KB) * (kBKV * kD * 2), 0)
-#define DOE_PF_LOAD_V(KB)                                                                            \
-    _Pragma("unroll") for (int i = 0; i < 4; ++i) rv[i] = __builtin_amdgcn_raw_buffer_load_b128(     \
-        vrsrc, v_voff + (uint32_t)i * 16u, (KB) * (kBKV * 2), 0)
-#define DOE_PF_STORE_K(BUF)                                                                          \
-    _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                                  \
-        const int gi = tid + 256 * i;                                                                \
-        *reinterpret_cast<u32x4 *>(&Ks[BUF][(gi >> 4) * kKRow + (gi & 15) * 8]) = rk[i];             \
+        (void *)(a.v + (size_t)kvh * a.kv_stride * kD), (short)0, a.kv_len * (kD * 2), 0x00020000);
+    // wave w stages rows 4 NP w + 4 i + lane / 16 of K, thread t row 4 W i + t / 16 of V
+    uint32_t k_voff[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int key = 4 * NP * wave + 4 * i + (lane >> 4);
+        k_voff[i] = (uint32_t)(key * 256 + (((lane & 15) ^ (key & 15)) * 16));
     }
-#define DOE_PF_STORE_V(BUF)                                                                          \
-    _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                                  \
-        /* rows are 8-byte aligned: two b64 stores */                                                \
-        u32x2 *dst = reinterpret_cast<u32x2 *>(&Vt[BUF][vd * kVRow + 32 * vh + 8 * i]);              \
-        dst[0] = u32x2{rv[i].x, rv[i].y};                                                            \
-        dst[1] = u32x2{rv[i].z, rv[i].w};                                                            \
+    const uint32_t v_voff = (uint32_t)tid * 16u;  // + kStep i
+    const uint32_t v_lds = (uint32_t)((tid >> 4) * 256 + ((tid & 15) ^ (4 * ((tid >> 4) & 3))) * 16);  // + kStep i
+    auto load_k = [&](int kb, int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i)
+            load_lds16(krsrc, lds + slot * kBlock + (NP * wave + i) * 1024, k_voff[i],
+                       (uint32_t)min(kb, nkb - 1) * (uint32_t)kBlock);
+    };
+    u32x4 rv[NP];
+    auto load_v = [&](int i, int kb) __attribute__((always_inline)) {
+        rv[i] = __builtin_amdgcn_raw_buffer_load_b128(vrsrc, v_voff + (uint32_t)(i * kStep),
+                                                      (uint32_t)min(kb, nkb - 1) * (uint32_t)kBlock, 0);
+    };
+    auto convert_v = [&](int i, int part) __attribute__((always_inline)) {
+        rv[i][2 * part] = bf16pair_to_f16pair(rv[i][2 * part]);
+        rv[i][2 * part + 1] = bf16pair_to_f16pair(rv[i][2 * part + 1]);
+    };
+    auto store_v = [&](int i, int slot) __attribute__((always_inline)) {
+        *reinterpret_cast<u32x4 *>(lds + (kKRing + slot) * kBlock + v_lds + i * kStep) = rv[i];
+    };
+    // K operand s: key 32 kh + lr, dims 16 s + 8 lg (chunk 2 s + lg)
+    const uint32_t k_off = (uint32_t)((32 * kh + lr) * 256 + ((lg ^ (lr & 15)) * 16));
+    auto kfrag = [&](int s, uint32_t slot_off) __attribute__((always_inline)) {
+        return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + ((k_off ^ (uint32_t)(32 * s)) + slot_off)));
+    };
+    // V^T operand of dims 32 t .., step st: keys 32 kh + 16 st + 4 lg + 0..3 and
+    // + 8, dim 32 t + lr; a lane's address is that of a quad of one key's dims
+    uint32_t va[4];
+    {
+        const int key = 4 * lg + ((lane >> 2) & 3), c0 = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            va[t] = (uint32_t)(kKRing * kBlock + (32 * kh + key) * 256 + ((c0 + 4 * t) ^ (4 * (key & 3))) * 16 + (lane & 1) * 8);
     }
+    auto vfrag = [&](int t, int st, uint32_t slot_off) __attribute__((always_inline)) {
+        const uint8_t *p = lds + (va[t] + slot_off) + st * 4096;
+        const s16x4 v0 = read_tr((lds_s16x4 *)p), v1 = read_tr((lds_s16x4 *)(p + 2048));
+        return __builtin_bit_cast(half8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
 
+    const float16v zero = {0.0f};
     float16v o[4];
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] = 0.0f;
-    float m_i = -INFINITY, l_i = 0.0f;
-    if (nkb == 0) {
-        // no visible keys (only for rows past q_len): nothing to accumulate
-    } else {
-    // blocks [0, nkb_full) hold only keys every query of the workgroup sees
-    const int vis_all = a.causal ? min(a.kv_len, a.start_pos + q0 + 1) : a.kv_len;
-    const int nkb_full = min(nkb, vis_all / kBKV);
+    for (int t = 0; t < 4; ++t) o[t] = zero;
+    float m_i = -INFINITY, l_i = 0.0f, bmax = -INFINITY;
+    // key blocks [0, nkb_full) hold only keys that every query of the workgroup sees
+    const int nkb_full = min(nkb, (a.causal ? min(a.kv_len, a.start_pos + q0 + 1) : a.kv_len) / kBKV);
     const half2v ones = {(_Float16)1.0f, (_Float16)1.0f};
+    // score r: key 32 kh + (r % 4) + 8 (r / 4) + 4 lg of the block
+    auto masked = [&](float x, int r, int kb) __attribute__((always_inline)) {
+        return kb * kBKV + 32 * kh + (r & 3) + 8 * (r >> 2) + 4 * lg < limit ? x : -INFINITY;
+    };
 
-    // S^T of the block in Ks[buf]: D[i] = key (i%4) + 8(i/4) + 4 lg of half kb2, query lr
-    auto s_mfmas = [&](float16v (&st)[2], const int buf) __attribute__((always_inline)) {
+    // Prologue: K(0 .. 2) and V(0), V(1) are loaded, V(0) converted, S(0) formed
+    load_k(0, 0);
 #pragma unroll
-        for (int kb2 = 0; kb2 < 2; ++kb2) {
+    for (int i = 0; i < NP; ++i) load_v(i, 0);
+    load_k(1, 1);
+    load_k(2, 2);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) st[kb2][r] = 0.0f;
+    for (int i = 0; i < NP; ++i) {
+        convert_v(i, 0);
+        convert_v(i, 1);
+        store_v(i, 0);
+    }
 #pragma unroll
-            for (int s = 0; s < 8; ++s) {
-                const bf16x8 kf = __builtin_bit_cast(
-                    bf16x8, *reinterpret_cast<const u32x4 *>(&Ks[buf][(32 * kb2 + lr) * kKRow + 16 * s + 8 * lg]));
-                st[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], st[kb2], 0, 0, 0);
-            }
+    for (int i = 0; i < NP; ++i) load_v(i, 1);
+    wait_barrier<3 * NP>();
+    float16v sa, sb;
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+        sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfrag(s, 0), qf[s], s ? sa : zero, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        if (nkb_full == 0) sa[r] = masked(sa[r], r, 0);
+        bmax = fmaxf(bmax, sa[r]);
+    }
+    bmax = halves_max(bmax);
+    wait_barrier<2 * NP>();  // K(1) has landed; every wave has read K(0)
+
+    // Iteration kb: sc holds block kb's scores, sn receives block kb + 1's (mode
+    // 0: none of them masked, 1: masked, 2: there is none).  At its start K(kb +
+    // 1) and V(kb) are in LDS, K(kb + 2) and V(kb + 1) under way; it issues K(kb
+    // + 3) and, as V(kb + 1)'s registers come free, V(kb + 2) (past the last: the
+    // last again, never used).  One wave per SIMD: what the vector unit does is
+    // dealt out between the MFMAs, each step its own scheduling region.
+    uint32_t ks_next = kBlock;  // K(kb + 1)'s place in the ring
+    int ks_load = 0;            // K(kb + 3)'s
+    auto iter = [&](const int kb, const int mode, float16v &sc, float16v &sn) __attribute__((always_inline)) {
+        const uint32_t vs = (uint32_t)(kb & 1) * kBlock;
+        bf16x8 kf[4];
+        if (mode != 2) {
+#pragma unroll
+            for (int s = 0; s < 3; ++s) kf[s] = kfrag(s, ks_next);
+            load_k(kb + 3, ks_load);
         }
-    };
-    // masks block kbb's scores (keys >= limit -> -inf) and returns their raw max
-    // over the query's two lane halves (the scale is positive: max commutes)
-    auto block_max = [&](float16v (&st)[2], const int kbb, const bool mask) __attribute__((always_inline)) {
-        float bmax = -INFINITY;
-#pragma unroll
-        for (int kb2 = 0; kb2 < 2; ++kb2)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                if (mask) {
-                    const int key = kbb * kBKV + 32 * kb2 + (r & 3) + 8 * (r >> 2) + 4 * lg;
-                    if (key >= limit) st[kb2][r] = -INFINITY;
-                }
-                bmax = fmaxf(bmax, st[kb2][r]);
-            }
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(bmax), __float_as_uint(bmax), false, false);
-        return fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    };
-
-    DOE_PF_LOAD_K(0);
-    DOE_PF_LOAD_V(0);
-    DOE_PF_STORE_K(0);
-    DOE_PF_STORE_V(0);
-    DOE_PF_LOAD_K(min(1, nkb - 1));
-    DOE_PF_STORE_K(1);
-    __syncthreads();
-    float16v sc[2];
-    s_mfmas(sc, 0);
-    float bmax_c = block_max(sc, 0, nkb_full == 0);
-    __syncthreads();  // every wave has read K(0) before iteration 0 overwrites Ks[0]
-
-    // iteration kb: sc holds block kb's scores, sn receives block kb + 1's
-    auto iter = [&](const int kb, const bool mask_next, float16v(&sc)[2], float16v(&sn)[2]) __attribute__((always_inline)) {
-        const int vb = kb & 1, kn = (kb + 1) & 1;
-        DOE_PF_LOAD_K(min(kb + 2, nkb - 1));
-        DOE_PF_LOAD_V(min(kb + 1, nkb - 1));
-        // running max for block kb (raised only past m + 8: P <= 2^8)
-        const float mb = bmax_c * a.scale_log2;
+        const float mb = bmax * a.scale_log2;
         if (__builtin_amdgcn_ballot_w64(mb > m_i + kLazy) != 0) {  // wave-uniform
             const float m_new = fmaxf(m_i, mb);
             const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_i - m_new);
             m_i = m_new;
             l_i *= alpha;
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+                for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
         }
         const float nm = m_i == -INFINITY ? 0.0f : -m_i;
-        // The next block's scores under this block's softmax: MFMA i of S^T
-        // (half i % 2, dims 16 (i / 2)) with the K fragment read four MFMAs
-        // ahead and score pair i of this block turned into f16 P.  Each step is
-        // its own scheduling region, so the exp2s stay between the MFMAs.
-#pragma unroll
-        for (int kb2 = 0; kb2 < 2; ++kb2)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sn[kb2][r] = 0.0f;
-        auto kfrag = [&](const int i) __attribute__((always_inline)) {
-            return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(
-                                                  &Ks[kn][(32 * (i & 1) + lr) * kKRow + 16 * (i >> 1) + 8 * lg]));
-        };
-        constexpr int kAhead = 4;  // fragment reads this many MFMAs ahead of their use
-        bf16x8 kf[kAhead + 1];
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i) kf[i] = kfrag(i);
-        half8 pf[4];
-        float psum = 0.0f;
-        // score pair i: slice i / 4, slots 2 (i % 4), 2 (i % 4) + 1.  Its exp2s
-        // are issued in step i and converted / summed in step i + 1, so no
-        // instruction waits on a just-issued transcendental (the wave issues
-        // in order: such a wait would hold back the next MFMA).
+        // Score pair p (step p / 4 of P V): its exp2s are issued in one step and
+        // converted and summed in the next, so that nothing waits on a
+        // just-issued transcendental (the wave issues in order).
+        half8 pf[2];
         float pp0 = 0.0f, pp1 = 0.0f;
-        auto finish_pair = [&](const int i) __attribute__((always_inline)) {
-            const int s4 = i >> 2, j = 2 * (i & 3);
-            const half2v h = {(_Float16)pp0, (_Float16)pp1};
-            psum = __builtin_amdgcn_fdot2(h, ones, psum, false);
-            pf[s4][j] = h[0];
-            pf[s4][j + 1] = h[1];
+        auto finish_pair = [&](int p) __attribute__((always_inline)) {
+            const half2v h = __builtin_convertvector((float2v{pp0, pp1}), half2v);
+            l_i = __builtin_amdgcn_fdot2(h, ones, l_i, false);
+            pf[p >> 2][2 * (p & 3)] = h[0];
+            pf[p >> 2][2 * (p & 3) + 1] = h[1];
         };
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            sn[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i % (kAhead + 1)], qf[i >> 1], sn[i & 1], 0, 0, 0);
-            if (i + kAhead < 16) kf[(i + kAhead) % (kAhead + 1)] = kfrag(i + kAhead);
-            const int s4 = i >> 2, j = 2 * (i & 3);
-            const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[s4 >> 1][8 * (s4 & 1) + j], a.scale_log2, nm));
-            const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[s4 >> 1][8 * (s4 & 1) + j + 1], a.scale_log2, nm));
-            if (i > 0) finish_pair(i - 1);
+        auto do_pair = [&](int p) __attribute__((always_inline)) {
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[2 * p], a.scale_log2, nm));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[2 * p + 1], a.scale_log2, nm));
+            if (p > 0) finish_pair(p - 1);
             pp0 = p0;
             pp1 = p1;
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        finish_pair(15);
-        l_i += psum;
-        // O^T[d][q] += V^T[d][keys] . P^T[keys][q] (slot 8 lg + j of slice s4 is key
-        // 32 (s4/2) + 16 (s4%2) + 4 lg + (j%4) + 8 (j/4) -- the D layout of S^T),
-        // MFMA i = (slice i / 4, dims 32 (i % 4)) with its V^T fragment read four
-        // MFMAs ahead, under the next block's mask and max.
-        auto vfrag = [&](const int i) __attribute__((always_inline)) {
-            const int s4 = i >> 2, db = i & 3;
-            const _Float16 *vr = &Vt[vb][(32 * db + lr) * kVRow + 32 * (s4 >> 1) + 16 * (s4 & 1) + 4 * lg];
-            const u32x2 v0 = *reinterpret_cast<const u32x2 *>(vr);
-            const u32x2 v1 = *reinterpret_cast<const u32x2 *>(vr + 8);
-            return __builtin_bit_cast(half8, u32x4{v0.x, v0.y, v1.x, v1.y});
         };
-        half8 vf[kAhead + 1];
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i) vf[i] = vfrag(i);
-        float bm[2] = {-INFINITY, -INFINITY};  // two independent chains
+        constexpr int kEarly = 5;  // pairs under Q K; the other three under P V's first step
+        half8 vf[4];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            o[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i % (kAhead + 1)], pf[i >> 2], o[i & 3], 0, 0, 0);
-            if (i + kAhead < 16) vf[(i + kAhead) % (kAhead + 1)] = vfrag(i + kAhead);
-            // scores 2i, 2i + 1 of the next block: half i / 8, slots 2 (i % 8), + 1
+        for (int i = 0; i < 8; ++i) {
+            if (mode != 2) {
+                sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i & 3], qf[i], i ? sn : zero, 0, 0, 0);
+                if (i + 3 < 8) kf[(i + 3) & 3] = kfrag(i + 3, ks_next);
+            }
+            if (i >= 5) vf[i - 5] = vfrag(i - 5, 0, vs);
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int kb2 = i >> 3, r = 2 * (i & 7) + e;
-                if (mask_next) {
-                    const int key = (kb + 1) * kBKV + 32 * kb2 + (r & 3) + 8 * (r >> 2) + 4 * lg;
-                    if (key >= limit) sn[kb2][r] = -INFINITY;
+            for (int p = i * kEarly / 8; p < (i + 1) * kEarly / 8; ++p) do_pair(p);
+            if (mode != 2) __builtin_amdgcn_sched_barrier(0);
+        }
+        float bm[2] = {-INFINITY, -INFINITY};
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {  // step i / 4, dims 32 (i % 4)
+            o[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i & 3], pf[i >> 2], o[i & 3], 0, 0, 0);
+            if (i + 3 < 8) vf[(i + 3) & 3] = vfrag((i + 3) & 3, (i + 3) >> 2, vs);
+            if (i < 8 - kEarly) do_pair(kEarly + i);
+            if (i == 8 - kEarly) finish_pair(7);
+            if (mode != 2 && i >= 4) {  // V(kb + 1), and the next block's mask and max
+                constexpr int kPer = 4 / NP;  // PV steps per piece
+                const int c = (i - 4) / kPer;
+#pragma unroll
+                for (int part = 0; part < 2 / kPer; ++part) convert_v(c, kPer == 2 ? i & 1 : part);
+                if ((i - 4) % kPer == kPer - 1) {
+                    store_v(c, (kb + 1) & 1);
+                    load_v(c, kb + 2);
                 }
-                bm[e] = fmaxf(bm[e], sn[kb2][r]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = 4 * (i - 4) + e;
+                    if (mode == 1) sn[r] = masked(sn[r], r, kb + 1);
+                    bm[e & 1] = fmaxf(bm[e & 1], sn[r]);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        float bmax_n;
-        {
-            const float bmm = fmaxf(bm[0], bm[1]);
-            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(bmm), __float_as_uint(bmm), false, false);
-            bmax_n = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+        if (mode != 2) {
+            bmax = halves_max(fmaxf(bm[0], bm[1]));
+            ks_next = ks_next == (kKRing - 1) * kBlock ? 0 : ks_next + kBlock;
+            ks_load = ks_load == kKRing - 1 ? 0 : ks_load + 1;
+            wait_barrier<2 * NP>();  // K(kb + 2) has landed, V(kb + 1) is written
         }
-        DOE_PF_STORE_K(vb);  // K(kb + 2): K(kb) was read before the previous barrier
-        DOE_PF_STORE_V(kn);  // V(kb + 1): V(kb - 1) likewise
-        __syncthreads();
-        bmax_c = bmax_n;
     };
-    float16v sn[2];
     int kb = 0;
     for (; kb + 2 < nkb_full; kb += 2) {  // two iterations whose next blocks need no mask
-        iter(kb, false, sc, sn);
-        iter(kb + 1, false, sn, sc);
+        iter(kb, 0, sa, sb);
+        iter(kb + 1, 0, sb, sa);
     }
-    for (; kb < nkb; ++kb) {  // the rest (a mask on blocks every query sees is a no-op)
-        iter(kb, true, sc, sn);
-#pragma unroll
-        for (int kb2 = 0; kb2 < 2; ++kb2) sc[kb2] = sn[kb2];
+    for (; kb + 2 < nkb; kb += 2) {  // (a mask on blocks that every query sees is a no-op)
+        iter(kb, 1, sa, sb);
+        iter(kb + 1, 1, sb, sa);
     }
+    if (kb + 1 < nkb) {
+        iter(kb, 1, sa, sb);
+        iter(kb + 1, 2, sb, sa);
+    } else {
+        iter(kb, 2, sa, sb);
     }
-#undef DOE_PF_LOAD_K
-#undef DOE_PF_LOAD_V
-#undef DOE_PF_STORE_K
-#undef DOE_PF_STORE_V
 
-    if (qi >= a.q_len) return;
-    const auto lsw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_i), __float_as_uint(l_i), false, false);
-    const float l_tot = __uint_as_float(lsw[0]) + __uint_as_float(lsw[1]);
-    const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    const size_t obase = ((size_t)qi * a.hq + h) * kD;
+    // Merge: the waves of the two key halves (w, w ^ (W / 2)) hold the same queries; each
+    // passes its lanes' sums of the other's half of the dims on
+    wait_barrier<0>();  // every wave is done with the rings, every load has landed
+    const float l = halves_sum(l_i);
+    float4 *xo = reinterpret_cast<float4 *>(lds);
+    float2 *xm = reinterpret_cast<float2 *>(lds + kExchange);
+    auto finish = [&](const int t0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+        for (int i = 0; i < 8; ++i) {
+            const float16v &ot = o[(2 - t0) + (i >> 2)];
+            const int g = 4 * (i & 3);
+            xo[(wave * 8 + i) * 64 + lane] = make_float4(ot[g], ot[g + 1], ot[g + 2], ot[g + 3]);
+        }
+        xm[wave * 64 + lane] = make_float2(m_i, l);
+        wait_barrier<0>();
+        const float2 p = xm[(wave ^ (W / 2)) * 64 + lane];
+        const float M = fmaxf(m_i, p.x);
+        const float f0 = m_i == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_i - M);
+        const float f1 = p.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(p.x - M);
+        const float lt = l * f0 + p.y * f1;
+        const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+        const float i0 = f0 * inv, i1 = f1 * inv;
+        if (qi >= a.q_len) return;
+        const size_t obase = ((size_t)qi * a.hq + head) * kD;
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-            const int d0 = 32 * db + 8 * r4 + 4 * lg;
-            const float v0 = o[db][4 * r4] * inv, v1 = o[db][4 * r4 + 1] * inv;
-            const float v2 = o[db][4 * r4 + 2] * inv, v3 = o[db][4 * r4 + 3] * inv;
+        for (int i = 0; i < 8; ++i) {
+            const float16v &ot = o[t0 + (i >> 2)];
+            const int g = 4 * (i & 3), d0 = 32 * (t0 + (i >> 2)) + 8 * (i & 3) + 4 * lg;
+            const float4 w = xo[((wave ^ (W / 2)) * 8 + i) * 64 + lane];
+            const float v0 = ot[g] * i0 + w.x * i1, v1 = ot[g + 1] * i0 + w.y * i1;
+            const float v2 = ot[g + 2] * i0 + w.z * i1, v3 = ot[g + 3] * i0 + w.w * i1;
             if (a.out_bf16) {
-                const u32x2 w = {(uint32_t)f32_to_bf16_rne(v0) | ((uint32_t)f32_to_bf16_rne(v1) << 16),
+                const u32x2 b = {(uint32_t)f32_to_bf16_rne(v0) | ((uint32_t)f32_to_bf16_rne(v1) << 16),
                                  (uint32_t)f32_to_bf16_rne(v2) | ((uint32_t)f32_to_bf16_rne(v3) << 16)};
-                *reinterpret_cast<u32x2 *>(reinterpret_cast<uint16_t *>(a.out) + obase + d0) = w;
+                *reinterpret_cast<u32x2 *>(reinterpret_cast<uint16_t *>(a.out) + obase + d0) = b;
             } else {
                 *reinterpret_cast<float4 *>(reinterpret_cast<float *>(a.out) + obase + d0) = make_float4(v0, v1, v2, v3);
             }
         }
+    };
+    if (kh == 0)
+        finish(0);
+    else
+        finish(2);
 }
 
-// Library-owned workspace (grow-only) for the f16 V^T copy.
-std::mutex g_ws_mu;
-void *g_ws = nullptr;
-size_t g_ws_bytes = 0;
+template <int W>
+int launch(const PrefillArgs &a, int64_t blocks, hipStream_t st) {
+    static const hipError_t attr_rc = hipFuncSetAttribute((const void *)attn_prefill_kernel<W>,
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    DOE_HIP_CHECK(attr_rc);
+    hipLaunchKernelGGL((attn_prefill_kernel<W>), dim3((unsigned)blocks), dim3(64 * W), kLds, st, a);
+    DOE_LAUNCH_CHECK("attn_prefill_kernel");
+    return DOE_OK;
+}
 
 }  // namespace
 
@@ -411,6 +430,7 @@ int doe_attn_prefill(const uint16_t *q, const uint16_t *k, const uint16_t *v, vo
     PrefillArgs a;
     a.q = q;
     a.k = k;
+    a.v = v;
     a.out = out;
     a.hq = (int)num_heads;
     a.hkv = (int)num_kv_heads;
@@ -420,7 +440,15 @@ int doe_attn_prefill(const uint16_t *q, const uint16_t *k, const uint16_t *v, vo
     a.start_pos = (int)start_pos;
     a.causal = causal ? 1 : 0;
     a.out_bf16 = out_bf16 ? 1 : 0;
-    a.nqb = (int)((q_len + kBQ - 1) / kBQ);
+    a.pair = (num_heads / num_kv_heads) % 2 == 0;
+    a.cols = (int)(a.pair ? num_heads / 2 : num_heads);
+    const int64_t rows = a.pair ? 2 * q_len : q_len;  // of a column
+    // Eight waves once the four-wave workgroups (two per CU) come to well over one
+    // round: half of the staging, which then counts (704 of them 30.3 against
+    // 32.7 us, 1024 56 against 60, back to back); up to there four: more, shorter
+    // workgroups (560: 23.1 against 24.6; 512: 36.7 against 39.5; 96: 24 against 33)
+    const bool wide = (rows + 63) / 64 * a.cols > 640;
+    a.units = (int)(wide ? (rows + 127) / 128 : (rows + 63) / 64);
     a.scale_log2 = scale * 1.4426950408889634f;
     hipStream_t st = (hipStream_t)stream;
     if (kv_len == 0) {
@@ -428,30 +456,9 @@ int doe_attn_prefill(const uint16_t *q, const uint16_t *k, const uint16_t *v, vo
         const size_t bytes = (size_t)q_len * num_heads * kD * (out_bf16 ? 2 : 4);
         return doe::fill_bytes_async(out, 0, bytes, st);
     }
-    const int64_t blocks = (int64_t)a.nqb * a.hq;
+    const int64_t blocks = (int64_t)a.units * a.cols;
     DOE_REQUIRE(blocks <= 0x7fffffff, DOE_E_UNSUPPORTED, "too many blocks");
-    const int64_t nkb_all = (kv_len + kBKV - 1) / kBKV;
-    a.kv_pad = (int)(nkb_all * kBKV);
-    const size_t need = (size_t)num_kv_heads * kD * (size_t)a.kv_pad * sizeof(_Float16);
-    _Float16 *vt;
-    {
-        std::lock_guard<std::mutex> lk(g_ws_mu);
-        if (g_ws_bytes < need) {
-            doe::retire_workspace(g_ws);  // queued kernels and captured graphs may still use it
-            g_ws = nullptr;
-            g_ws_bytes = 0;
-            DOE_HIP_CHECK(hipMalloc(&g_ws, need));
-            g_ws_bytes = need;
-        }
-        vt = (_Float16 *)g_ws;
-    }
-    a.vt = vt;
-    hipLaunchKernelGGL(v_to_f16t_kernel, dim3((unsigned)nkb_all, (unsigned)num_kv_heads), dim3(256), 0, st, v, vt,
-                       a.kv_len, a.kv_stride, a.kv_pad);
-    DOE_LAUNCH_CHECK("v_to_f16t_kernel");
-    hipLaunchKernelGGL(attn_prefill_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a);
-    DOE_LAUNCH_CHECK("attn_prefill_kernel");
-    return DOE_OK;
+    return wide ? launch<8>(a, blocks, st) : launch<4>(a, blocks, st);
 }
 
 }  // extern "C"

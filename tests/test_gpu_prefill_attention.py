@@ -134,6 +134,26 @@ def test_prefill_more_workgroups_than_slots(dev, ora):
         assert rel_l2(got[r0:r1], want[r0:r1]) <= TOL, (r0, r1)
 
 
+# Four-wave workgroups (64 rows) and, past 640 of those, eight-wave ones (128):
+# one or two heads to a workgroup, the last rows and keys partial, a cache longer
+# than the keys, keys before the prompt, all keys visible.  The contract's bound.
+@pytest.mark.parametrize("hq,hkv,s,start,causal", [
+    (6, 2, 95, 0, True), (6, 2, 33, 70, True), (2, 1, 31, 1, True), (4, 1, 161, 64, True), (2, 2, 66, 63, False),
+    (64, 32, 675, 0, True), (63, 21, 705, 33, True), (64, 64, 650, 5, False)])
+def test_prefill_workgroup_widths(dev, ora, hq, hkv, s, start, causal):
+    rng = np.random.default_rng(hq + s)
+    kv, stride = start + s, start + s + 3
+    q = to_bf16(rng.standard_normal((s, hq, D), dtype=np.float32))
+    k = to_bf16(rng.standard_normal((hkv, stride, D), dtype=np.float32))
+    v = to_bf16(rng.standard_normal((hkv, stride, D), dtype=np.float32))
+    got = run(q, k, v, hq, hkv, s, kv, stride, start, 0.1, causal)
+    assert np.isfinite(got).all()
+    rows = [(0, s)] if s < 200 else [(0, 2), (63, 66), (127, 130), (s - 3, s)]
+    for r0, r1 in rows:
+        want = oracle(ora, q, k, v, hq, hkv, s, kv, stride, start, 0.1, causal, rows=(r0, r1))
+        assert rel_l2(got[r0:r1], want[r0:r1]) <= TOL, (r0, r1)
+
+
 def test_prefill_graph_replays(dev):
     # replays of one captured call (the V^T pre-pass and the attention kernel),
     # with eager calls in between, all reproduce the eager result exactly
