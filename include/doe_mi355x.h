@@ -250,9 +250,10 @@ int doe_q4k_gemm(const uint16_t *a_bf16, const void *b_q4k, float *c, int64_t m,
                  int64_t k, doe_stream_t stream);
 
 /* doe_q4k_gemm with f32 activations a [m][k] (a prompt's f32 hidden states,
- * the step graphs' af32 activation format): each row is scaled by a power of
- * two and rounded once to f16 (11 significant bits) by the pre-pass, then
- * the same matrix-core GEMM; the same workspace rule. */
+ * the step graphs' af32 activation format), f32-accurate: each row is scaled by
+ * a power of two and carried as f16 hi + lo, the weights as their stored
+ * integers with the block scales applied to f32 sums (2-5e-7 from float64 at
+ * the prompt shapes); the same workspace rule, four bytes per element of a. */
 int doe_q4k_gemm_f32(const float *a, const void *b_q4k, float *c, int64_t m, int64_t n, int64_t k,
                      doe_stream_t stream);
 /* The same GEMM over Q8_0 rows (the `matmul` op with quantFormat q8_0 at
@@ -667,7 +668,7 @@ int doe_decode_advance(int32_t *state, int32_t *token, int32_t *ids, int64_t max
  * "int4_gemv.xcd" (1: workgroup ids in plain order, not a row block's K
  * ranges grouped on one XCD), "q8_0_gemv.rows" (1, 2 or 4 rows per wave group), "q8_0_gemv.depth" (1 or
  * 2 blocks loaded ahead), "attn_mq.splits" (1..16 key splits of the
- * multi-query attention), "attn_decode.splits",
+ * 16-query form of the multi-query attention, at any head_dim), "attn_decode.splits",
  * "attn_decode.waves" (4: narrow workgroups; 8 or 16: the wide short-context
  * workgroup where the head shape allows it), "attn_decode.combine" (1: the
  * block-reduction split combine instead of the one-wave-per-column form),
