@@ -654,8 +654,11 @@ namespace doe {
 // most 32: their partials are written and summed once more), by the least of
 //   blocks of 256 K on the busiest CU x us per block + the partials' traffic.
 // A CU takes 3.6 us per block of a 128-row Q4_K tile with one workgroup or two
-// (4.7 Q8_0), 2.1 of a 64-row one (3.3); the summing pass costs 3.5 us and its
-// bytes at 4 TB/s.  Measured (Q4_K, us, with the rule / the other tile height /
+// (5.0 Q8_0, and 0.3 of a block to fill the pipeline), 2.1 of a 64-row one (3.3);
+// the summing pass costs 3.5 us and its bytes at 4 TB/s (Q8_0 8: with 4, three
+// splits of 600 x 4096 x 2304, 48.6 us, lost to one, 52.8; so 1000 x 2304 x 9216
+// 146 -> 142 and the norm + GeGLU of 128 x 18432 x 2304 51.4 -> 49.1.  Q4_K at 8
+// would split the latter, 39 -> 43).  Measured (Q4_K, us, with the rule / the other tile height /
 // two workgroups per CU filled with splits): 128 x 18432 x 2304 39 / 40 / 43
 // (128 rows, one split), 128 x 4096 x 2304 20 / 24 / 28 (64 rows, three),
 // 512 x 2304 x 9216 65 / 92 / 75 (128 rows, three), 20 x 18432 x 2304 23.5
@@ -665,12 +668,12 @@ GemmF32Plan gemm_f32_plan(int64_t m, int64_t n, int64_t k, int fmt, int num_cus)
     const int64_t nblk = (padded_k(k, fmt) + 255) / 256;
     double best = 0.0;
     for (int rows = 64; rows <= 128; rows += 64) {
-        const double block_us = rows == 64 ? (fmt == 0 ? 2.1 : 3.3) : (fmt == 0 ? 3.6 : 4.7);
+        const double block_us = rows == 64 ? (fmt == 0 ? 2.1 : 3.3) : (fmt == 0 ? 3.6 : 5.0);
         const int64_t tiles = ((m + rows - 1) / rows) * ((n + 127) / 128);
         for (int64_t want = 1; want <= 32 && want <= nblk && (want == 1 || tiles * want <= 3 * num_cus); ++want) {
             const int64_t per = (nblk + want - 1) / want, splits = (nblk + per - 1) / per;
-            double us = (double)((tiles * splits + num_cus - 1) / num_cus) * (double)per * block_us;
-            if (splits > 1) us += 3.5 + (double)splits * (double)(m * n) * 8e-6 / 4.0;
+            double us = (double)((tiles * splits + num_cus - 1) / num_cus) * ((double)per + (fmt == 0 ? 0.0 : 0.3)) * block_us;
+            if (splits > 1) us += 3.5 + (double)splits * (double)(m * n) * 8e-6 / (fmt == 0 ? 4.0 : 8.0);
             if (p.tile_rows == 0 || us < best) {
                 best = us;
                 p.tile_rows = rows;
