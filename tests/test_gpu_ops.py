@@ -69,6 +69,41 @@ def test_geglu_and_residual(dev, ora):
     assert np.array_equal(out.download(), ora.residual(g, u))
 
 
+@pytest.mark.parametrize("sigma", [0.3, 1.0, 3.0, 10.0])
+def test_geglu_accuracy_against_float64(dev, sigma):
+    # no further from 64 bits than the formula with a correctly rounded f32
+    # tanh (2-norm, and on the negative side by itself, where 1 + tanh cancels);
+    # 2 % for the tail of the sample; what lies below the f32 tanh's -1 is zero
+    rng = np.random.default_rng(int(10 * sigma))
+    n = 1 << 20
+    g = (rng.standard_normal(n) * sigma).astype(np.float32)
+    out = DeviceBuffer.empty((n,), np.float32)
+    ops.gelu_gated(up(g), up(np.ones(n, np.float32)), out, n)
+    got = out.download()
+    f = np.float32
+    inner = f(0.7978845608028654) * (g + f(0.044715) * g * g * g)
+    inner = np.clip(inner, f(-15), f(15))
+    by_tanh = f(0.5) * g * (f(1) + np.tanh(inner.astype(np.float64)).astype(f))
+    x = g.astype(np.float64)
+    want = 0.5 * x * (1 + np.tanh(np.clip(0.7978845608028654 * (x + 0.044715 * x ** 3), -15, 15)))
+    for part in (g == g, g < 0):
+        assert rel_l2(got[part], want[part]) <= 1.02 * rel_l2(by_tanh[part], want[part])
+    assert not got[inner < -9.03].any()
+
+
+def test_geglu_extremes(dev):
+    # zeros, the largest and smallest values, infinities and NaN, as 0.5 x (1 + tanh)
+    g = np.array([0.0, -0.0, 1e-38, -1e-38, 15.0, -15.0, 3e38, -3e38, np.inf, -np.inf, np.nan], np.float32)
+    out = DeviceBuffer.empty(g.shape, np.float32)
+    ops.gelu_gated(up(g), up(np.ones_like(g)), out, g.size)
+    got = out.download()
+    want = np.array([0.0, -0.0, 5e-39, -5e-39, 15.0, -0.0, 3e38, -0.0, np.inf, np.nan, np.nan], np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert np.allclose(got[ok], want[ok], rtol=1e-6, atol=2e-45)
+    assert np.array_equal(np.signbit(got[ok]), np.signbit(want[ok]))
+
+
 def test_rope_half_kv_rows_equals_rope_and_kv_write(dev, ora):
     # the prompt-row form in head order against doe_rope (same rotate-half
     # pairing and arithmetic) token by token and doe_kv_write: bit-exact
