@@ -7,14 +7,19 @@
 // integers it is stored as, exact in f16, so two products per step (a_hi b,
 // a_lo b) carry the full accuracy; the block scales are applied to the f32
 // sums afterwards:
-//   * Q4_K: b = sc q (6 x 4 bits, at most 945).  A 256-element block's sum is
-//     d sum(sc q x) - dmin sum_s m_s sum(x of sub-block s); the second term is
-//     one more MFMA per block, A's sub-block sums (f16 hi + lo, eight of each)
-//     against the eight 6-bit minima.
+//   * Q4_K: b = sc q - z (|b| < 2048), z the integer next to a sub-block's
+//     dmin m / d.  A 256-element block's sum is d sum(b x) + sum_s r_s sum(x of
+//     sub-block s), r = d z - dmin m: two more MFMAs per block, A's sub-block
+//     sums (f16 hi + lo, eight of each) against r as f16 hi + lo.  b d is the
+//     weight up to r, and |r| at most d: neither sum is larger than the
+//     result's own terms.  (With b = sc q and the minima in the second sum the
+//     two cancel wherever the activations of a row have a common sign.)
 //   * Q8_0: b = q (int8); a 32-element block's sum is d sum(q x).
-// 2-4e-7 from float64 at the prompt's shapes.  (Splitting the dequantised f32
-// weight into f16 hi + lo as well takes a third product per step and ~6 VALU
-// operations per weight instead of 1.1; 3.5-7.8e-7.)
+// Measured, rows of A with mean 0 to 30 deviations or after ReLU, K 2304 to
+// 13000: Q4_K 1.3-1.8e-7 from float64, Q8_0 1.0-1.4e-7.  (Splitting the
+// dequantised f32 weight into f16 hi + lo instead takes a third product per
+// step and ~6 VALU operations per weight instead of 1.1, and gives 1.9-2.6e-7;
+// b = sc q takes 4 % less time here, and gives 3.2e-7, with a mean 1.4-2.9e-6.)
 //
 // Layout.  The pre-pass writes A in operand order: per 32 rows and 32
 // elements of K four 1 KB fragments (step 0 hi, lo, step 1 hi, lo), each the
@@ -31,9 +36,9 @@
 // MFMAs (512 cycles), 16 fragment reads and ~25 VALU operations.
 // Measured (us per call, pre-pass and second pass included; the three-product
 // kernel with per-workgroup dequantisation that this replaced in brackets):
-// Q4_K norm + GeGLU 1000 x 18432 x 2304 180 (391: the matrix cores busy half
-// of 333 K cycles, the clock down to 1.8 GHz under them), Q8_0 333 x 2304 x
-// 9216 58 (83); 128-token calls are bound by the one or two waves per SIMD
+// Q4_K GeGLU 1000 x 18432 x 2304 188 (391: bound by the matrix cores, the
+// clock down to 1.8 GHz under them), Q8_0 333 x 2304 x 9216 58-62 (83);
+// 128-token calls are bound by the one or two waves per SIMD
 // that a short prompt gives.
 #include "gemm_f32.h"
 
@@ -229,15 +234,19 @@ __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t rsrc, void *ds
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)dst, 16, voff, soff, 0, 0);
 }
 
-// Eight f16 operands sc q 2^-14 from two nibble dwords: a nibble in bits 0..3
-// of a half is the subnormal q 2^-24 (scale sc 2^10), in bits 4..7 q 2^-20
-// (scale sc 2^6); every product is exact.
+// Eight f16 operands (sc q - z) 2^-14 from two nibble dwords: a nibble in bits
+// 0..3 of a half is the subnormal q 2^-24 (scale sc 2^10), in bits 4..7 q 2^-20
+// (scale sc 2^6); nz is -z 2^-14, every result is exact.
 template <bool HIGH>
-__device__ __forceinline__ half8 q4_operands(uint32_t w0, uint32_t w1, half2v sc) {
+__device__ __forceinline__ half8 q4_operands(uint32_t w0, uint32_t w1, half2v sc, half2v nz) {
     constexpr uint32_t mask = HIGH ? 0x00f000f0u : 0x000f000fu;
-    const uint32_t u[4] = {as_u32(as_h2(w0 & mask) * sc), as_u32(as_h2((w0 >> 8) & mask) * sc),
-                           as_u32(as_h2(w1 & mask) * sc), as_u32(as_h2((w1 >> 8) & mask) * sc)};
-    return __builtin_bit_cast(half8, u32x4{u[0], u[1], u[2], u[3]});
+    auto two = [&](uint32_t w) { return as_u32(__builtin_elementwise_fma(as_h2(w & mask), sc, nz)); };
+    return __builtin_bit_cast(half8, u32x4{two(w0), two(w0 >> 8), two(w1), two(w1 >> 8)});
+}
+// The 6-bit scales or minima of sub-blocks 2 c and 2 c + 1, from the two dwords of all eight.
+__device__ __forceinline__ half2v six_pair(const uint32_t (&v)[2], int c) {
+    const half2v k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
+    return as_h2(__builtin_amdgcn_perm(0x64646464u, v[c >> 1], c & 1 ? 0x04030402u : 0x04010400u)) - k1024;
 }
 // Eight f16 operands q from two dwords of int8 (1024 + (q + 128) - 1152).
 __device__ __forceinline__ half8 q8_operands(uint32_t w0, uint32_t w1) {
@@ -262,10 +271,10 @@ struct XTile {
 };
 
 // Q4_K: the loads a wave issues in stage u of a block: a fragment of A per
-// tile, a chunk of B at even stages, the block's sums at stage 0, a header at 2.
+// tile, a chunk of B at even stages, tile u's sums in the first TM, a header at 2.
 template <int TM>
 constexpr int q4_loads(int u) {
-    return TM + (u % 2 == 0) + (u == 0 ? TM : 0) + (u == 2);
+    return TM + (u % 2 == 0) + (u < TM) + (u == 2);
 }
 
 // FMT 0: Q4_K rows; 1: Q8_0 rows.
@@ -422,12 +431,15 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(XArgs g) {
         for (int u = 0; u < 3; ++u)
 #pragma unroll
             for (int i = 0; i < TM; ++i) load_a(2 * kc0 + u, u, i);
-        const u32x4 *sptr[TM];
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-            sptr[i] = g.sums + (size_t)min((m0 >> 5) + i, mtiles - 1) * (g.nsub >> 3) * 64 + lane;
-        const half2v k1024 = {(_Float16)1024.0f, (_Float16)1024.0f}, k64 = {(_Float16)64.0f, (_Float16)64.0f};
-        half2v sc[4];
+        const uint32_t sblocks = (uint32_t)g.nsub >> 3;
+        const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(g.sums + (size_t)(m0 >> 5) * sblocks * 64), (short)0,
+            (int)((uint32_t)min(TM, mtiles - (m0 >> 5)) * sblocks * 1024u), kBufFlags);
+        auto load_sums = [&](int i, int blk) __attribute__((always_inline)) {
+            return __builtin_amdgcn_raw_buffer_load_b128(
+                srsrc, 16u * lane, ((uint32_t)min(i, mtiles - 1 - (m0 >> 5)) * sblocks + (uint32_t)blk) * 1024u, 0);
+        };
+        half2v sc[4], nz[4];
         u32x4 raw;
         int bslot = 0;  // of the current chunk
         auto next_bslot = [&]() __attribute__((always_inline)) { return bslot == 2 ? 0 : bslot + 1; };
@@ -436,43 +448,83 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(XArgs g) {
             if (part == 0 && (u & 7) == 0) {
                 const u32x4 h = Bh((blk + (u >> 3)) & 1)[ncol];
                 const uint32_t sc6[2] = {h.y & 0x3f3f3f3fu, (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u)};
+                const uint32_t mn6[2] = {h.z & 0x3f3f3f3fu, ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u)};
                 const half2v up = {(_Float16)1024.0f, (_Float16)64.0f};
+                // z = m dmin / d to an integer in 0..1023 (the sum's ulp is 1; any
+                // integer is right, a near one makes r small)
+                const _Float16 t = (_Float16)(doe_half_bits_to_float(h.x >> 16) *
+                                              __builtin_amdgcn_rcpf(doe_half_bits_to_float(h.x)));
+                const half2v lo = {(_Float16)1024.0f, (_Float16)1024.0f}, hi = {(_Float16)2047.0f, (_Float16)2047.0f};
+                const half2v s14 = {(_Float16)-0x1p-14f, (_Float16)-0x1p-14f}, k = {(_Float16)0x1p-4f, (_Float16)0x1p-4f};
 #pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    sc[c] = (as_h2(__builtin_amdgcn_perm(0x64646464u, sc6[c >> 1], c & 1 ? 0x04030402u : 0x04010400u)) -
-                             k1024) * up;
+                for (int c = 0; c < 4; ++c) {
+                    sc[c] = six_pair(sc6, c) * up;
+                    half2v z = __builtin_elementwise_fma(six_pair(mn6, c), half2v{t, t}, lo);
+                    z = __builtin_elementwise_max(__builtin_elementwise_min(z, hi), lo);
+                    nz[c] = __builtin_elementwise_fma(z, s14, k);
+                }
             }
             if (part == 0 && (u & 1) == 0) raw = Bq(slot, lh)[ncol];
             if (part < TM - 2) return;
-            const half2v sv = sc[(u >> 1) & 3];
+            const half2v sv = sc[(u >> 1) & 3], zv = nz[(u >> 1) & 3];
             const int t = part - (TM - 2);  // the last two parts form step 0 and step 1
             const uint32_t w0 = t ? raw.z : raw.x, w1 = t ? raw.w : raw.y;
-            bf[t] = u & 1 ? q4_operands<true>(w0, w1, half2v{sv.y, sv.y}) : q4_operands<false>(w0, w1, half2v{sv.x, sv.x});
+            bf[t] = u & 1 ? q4_operands<true>(w0, w1, half2v{sv.y, sv.y}, half2v{zv.y, zv.y})
+                          : q4_operands<false>(w0, w1, half2v{sv.x, sv.x}, half2v{zv.x, zv.x});
         };
         // a block's sums are scaled as its last MFMAs end, a tile behind
-        float16v ms = zero;
-        float dl = 0.0f, dm = 0.0f;
+        float dl = 0.0f;
         auto scale_tile = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][r] = fmaf(ms[r], dm, fmaf(D[i][r], dl, acc[i][r]));
+            for (int r = 0; r < 16; ++r) acc[i][r] = fmaf(D[i][r], dl, acc[i][r]);
+        };
+        // r of the eight sub-blocks 2^(14 - E) (E: the block's largest dmin m and
+        // d z are below 2^E), formed a pair at a time in the first stages after the
+        // header's; tile i's sums are loaded in stage i and added in stage 3 + i
+        uint32_t rh[4], rl[4], mn6[2] = {0, 0};
+        float d_up = 0.0f, dmin_up = 0.0f, dm = 0.0f;
+        u32x4 sf[3];
+        float16v ms = zero;
+        auto remainders = [&](int blk, int c) __attribute__((always_inline)) {
+            if (c == 0) {
+                const u32x4 h = Bh(blk & 1)[ncol];
+                mn6[0] = h.z & 0x3f3f3f3fu;
+                mn6[1] = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
+                const float d = doe_half_bits_to_float(h.x), dmin = doe_half_bits_to_float(h.x >> 16);
+                dl = d * 16384.0f;
+                const int e = __builtin_amdgcn_frexp_expf(fmaxf(fabsf(d) * 1024.0f, fabsf(dmin) * 64.0f));
+                d_up = __builtin_amdgcn_ldexpf(d, 28 - e);  // (nz holds 2^-14)
+                dmin_up = __builtin_amdgcn_ldexpf(dmin, 14 - e);
+                dm = __builtin_amdgcn_ldexpf(1.0f, e - 8);  // (the sums hold 2^-6)
+            }
+            const half2v m = six_pair(mn6, c);
+            half2v top, low;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float r = -fmaf((float)nz[c][j], d_up, (float)m[j] * dmin_up);
+                top[j] = (_Float16)r;
+                low[j] = (_Float16)(r - (float)top[j]);
+            }
+            rh[c] = as_u32(top);
+            rl[c] = as_u32(low);
         };
         wait_barrier<2 * TM, 0>();
 #pragma unroll
         for (int i = 0; i < TM; ++i) operands(blk0, 0, 0, i);
         read_tile(0, 0);
         read_tile(0, 1);
-        half8 mn;
-        u32x4 sf[TM];
         for (int blk = blk0; blk < blk1; ++blk) {
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 const int kc = 4 * blk + (u >> 1), s = 8 * blk + u;
                 __builtin_amdgcn_sched_barrier(0);
                 switch (u) {
+                    case 0: case 6: wait_barrier<q4_loads<TM>(7), 8>(); break;
                     case 1: wait_barrier<q4_loads<TM>(0), 8>(); break;
+                    case 2: wait_barrier<q4_loads<TM>(1), 8>(); break;
                     case 3: wait_barrier<q4_loads<TM>(2), 8>(); break;
-                    case 5: case 7: wait_barrier<q4_loads<TM>(4), 8>(); break;
-                    default: wait_barrier<q4_loads<TM>(1), 8>(); break;
+                    case 4: wait_barrier<q4_loads<TM>(3), 8>(); break;
+                    default: wait_barrier<q4_loads<TM>(4), 8>(); break;
                 }
                 const half8 cur[2] = {bf[0], bf[1]};
 #pragma unroll
@@ -481,27 +533,25 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(XArgs g) {
                     load_a(min(s + 3, s1 - 1), (u + 3) & 3, i);
                     if (i == 0 && (u & 1) == 0) load_b4(min(kc + 3, kc1 - 1), bslot);
                     if (i == 1 && u == 2) load_h4(min(blk + 1, blk1 - 1));
-                    if (u == 0) sf[i] = sptr[i][(size_t)blk * 64];
+                    if (i == TM - 1 && u < TM) sf[u % 3] = load_sums(u, blk);
                     read_tile(u + (i + 2) / TM, (i + 2) % TM);
                     if (u == 0 && i == 0) scale_tile(TM - 1);
                     if (u == 7 && i > 0) scale_tile(i - 1);
                     mfma_tile(u, i, cur, u == 0);
-                    if (u == 7)
-                        ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, sf[i]), mn, zero, 0, 0, 0);
-                    operands(blk, u + 1, next_bslot(), i);
-                    if (u == 1 && i == 0) {
-                        const u32x4 h = Bh(blk & 1)[ncol];
-                        const uint32_t mn6[2] = {h.z & 0x3f3f3f3fu,
-                                                 ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u)};
-                        uint32_t mp[4];
+                    if (u >= 1 && (u - 1) * TM + i < 4) remainders(blk, (u - 1) * TM + i);
+                    if (u >= 3 && u < 3 + TM) {
+                        const half8 x = __builtin_bit_cast(half8, sf[u % 3]);
+                        if (i == 0) {
+                            ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                x, __builtin_bit_cast(half8, u32x4{rh[0], rh[1], rh[2], rh[3]}), zero, 0, 0, 0);
+                            ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                x, __builtin_bit_cast(half8, u32x4{rl[0], rl[1], rl[2], rl[3]}), ms, 0, 0, 0);
+                        } else if (i == TM / 2) {
 #pragma unroll
-                        for (int c = 0; c < 4; ++c)
-                            mp[c] = as_u32((as_h2(__builtin_amdgcn_perm(0x64646464u, mn6[c >> 1],
-                                                                        c & 1 ? 0x04030402u : 0x04010400u)) - k1024) * k64);
-                        mn = __builtin_bit_cast(half8, u32x4{mp[0], mp[1], mp[2], mp[3]});
-                        dl = doe_half_bits_to_float(h.x) * 16384.0f;
-                        dm = -doe_half_bits_to_float(h.x >> 16);
+                            for (int r = 0; r < 16; ++r) acc[u - 3][r] = fmaf(ms[r], dm, acc[u - 3][r]);
+                        }
                     }
+                    operands(blk, u + 1, next_bslot(), i);
                 }
                 if (u & 1) bslot = next_bslot();
             }

@@ -252,8 +252,11 @@ int doe_q4k_gemm(const uint16_t *a_bf16, const void *b_q4k, float *c, int64_t m,
 /* doe_q4k_gemm with f32 activations a [m][k] (a prompt's f32 hidden states,
  * the step graphs' af32 activation format), f32-accurate: each row is scaled by
  * a power of two and carried as f16 hi + lo, the weights as their stored
- * integers with the block scales applied to f32 sums (2-5e-7 from float64 at
- * the prompt shapes); the same workspace rule, four bytes per element of a. */
+ * integers (less an integer near each sub-block's minimum) with the block scales
+ * applied to f32 sums: 1.3-1.8e-7 from float64 at the prompt shapes, for rows of
+ * a with and without a mean.  A library-owned workspace of 4.2 bytes per element
+ * of a (rows padded to 32, k to 256) and, where K is split over the grid, 4 m n
+ * bytes per split, grown on demand (not during stream capture). */
 int doe_q4k_gemm_f32(const float *a, const void *b_q4k, float *c, int64_t m, int64_t n, int64_t k,
                      doe_stream_t stream);
 /* The same GEMM over Q8_0 rows (the `matmul` op with quantFormat q8_0 at

@@ -147,6 +147,48 @@ def test_gemm_f32_tile_edges(dev, ora, fmt, m, n, k):
         assert np.array_equal(h.download(), hw.download())
 
 
+def q4k_with_minima(rng, n, k, kind):
+    """Random Q4_K rows with the minima of one kind: "middle" of each sub-block's
+    range (dmin m = 7.5 d sc, what a quantizer of zero-mean weights writes),
+    "none" (every weight >= 0), "far" (dmin m up to 2000 d: every weight < 0),
+    "flat" (d = 0), "tiny" (d and dmin subnormal), "opposite" (dmin < 0)."""
+    nb = -(-k // 256)
+    w = rng.integers(0, 256, (n, nb, 144), np.uint8)
+    d = (np.abs(rng.standard_normal((n, nb))) * 2e-4 + 1e-5).astype(np.float16)
+    if kind == "tiny":
+        d = (rng.integers(1, 60, (n, nb)) * 2.0 ** -24).astype(np.float16)
+    factor = {"middle": 7.5, "none": 0.0, "far": 32.0, "flat": 7.5, "tiny": 7.5, "opposite": -7.5}[kind]
+    dmin = (factor * d.astype(np.float32)).astype(np.float16)
+    w[:, :, 0:2] = (d * (0 if kind == "flat" else 1)).astype(np.float16)[..., None].view(np.uint8)
+    w[:, :, 2:4] = dmin[..., None].view(np.uint8)
+    w[:, :, 8:12] = w[:, :, 4:8]  # minima equal to the scales
+    low = w[:, :, 12:16] & 15
+    w[:, :, 12:16] = low | (low << 4)
+    return w.reshape(n, -1)
+
+
+@pytest.mark.parametrize("minima", ["middle", "none", "far", "flat", "tiny", "opposite"])
+@pytest.mark.parametrize("m,n,k", [(70, 200, 2304), (500, 640, 9216), (33, 129, 1000)])
+def test_gemm_f32_one_sided_rows(dev, ora, m, n, k, minima):
+    # activations with a common sign (a mean, after ReLU, all equal), where the
+    # scales' and the minima's parts of a weight must not reach the sums apart.
+    # Bound: A's two f16 parts 2^-22; the 32 steps of a 256-element block and the
+    # k / 256 block sums round in f32, at random, relative to sums no larger than
+    # the result's terms.
+    rng = np.random.default_rng(m + k)
+    w = q4k_with_minima(rng, n, k, minima)
+    wf = ora.q4k_dequant_rowwise(w, n, k).astype(np.float64)
+    dw = up(w)
+    tol = 2.0 ** -22 + 2.0 ** -24 * (np.sqrt(32) + np.sqrt(k / 256))
+    z = rng.standard_normal((m, k), dtype=np.float32)
+    for name, a in (("mean", z + 3), ("relu", np.maximum(z, 0)), ("equal", np.full_like(z, -0.7)), ("zero mean", z)):
+        out = DeviceBuffer.empty((m, n), np.float32)
+        ops.matmul_gemm_f32_fused(up(a), dw, out, m, n, k, "q4k")
+        err = rel_l2(out.download(), a.astype(np.float64) @ wf.T)
+        print(f"[one-sided {name} {minima} {m}x{n}x{k}] {err:.2e} of {tol:.2e}", flush=True)
+        assert err <= tol, (name, err, tol)
+
+
 def test_gemm_prefill_config_sampled(dev, ora):
     # the 31B-class prefill shape: M=2048 tokens, K=5376, N=21504; the oracle
     # evaluates 2048 sampled entries (every row once, at a random column)
