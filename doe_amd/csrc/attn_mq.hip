@@ -14,10 +14,9 @@
 // writes zeros.
 //
 // Kernels.  head_dim 64 / 128 / 256 runs attn_mq32_kernel (below); head_dim 512
-// (whose Q and O do not fit one wave's registers there), caches past 2 GiB and
-// a forced key split attn_mq_kernel: one workgroup = 16 consecutive queries x
-// HG query heads of one KV
-// head (one wave per head), keys in blocks of 32 staged in LDS and shared by
+// (whose Q and O do not fit one wave's registers there) and caches of 2 GiB and
+// more (and attn_mq.queries = 16) attn_mq_kernel: one workgroup = 16
+// consecutive queries x HG query heads of one KV head (one wave per head), keys in blocks of 32 staged in LDS and shared by
 // the waves: K row-major for S = Q K^T and V transposed for O = P V, both on
 // v_mfma_f32_16x16x32_f16.  Q is f32: each query row is scaled by a power of
 // two (max near 2^14) and split into f16 hi + lo (~22 bits), so the scores
@@ -717,6 +716,7 @@ void *g_mq_ws = nullptr;
 size_t g_mq_ws_bytes = 0;
 int g_mq_cus = 0;
 int g_mq_splits = 0;
+int g_mq_queries = 0;  // 0 automatic, 16: attn_mq_kernel at any head_dim
 
 // The workspace of `splits` key splits' (o, m, l) in a.
 int split_workspace(MqArgs &a, int D) {
@@ -741,17 +741,31 @@ int launch_combine(const MqArgs &a, int D, hipStream_t st) {
     return DOE_OK;
 }
 
-// The 32-query kernel: caches that a 32-bit buffer offset reaches.  A short prompt over a long cache splits the keys over the grid, up
-// to one workgroup per CU and at least eight blocks (two per wave) each.
+// The 32-query kernel: caches that a 32-bit buffer offset reaches.  A short
+// prompt over a long cache splits the key blocks that its queries can see over
+// the grid, up to one workgroup per CU and at least eight blocks (two per wave)
+// each, at head_dim 256 two where there are 16 and more.  us, 17 queries, in
+// 1 / 2 / 4 / 8 / 16 splits: 8 / 4 heads x 256 over 145 keys 13.2 / 13.3 / 13.8
+// / 15.1 / 17.5, 517 keys 19.7 / 17.5 / 16.3 / 15.7 / 17.8, 2017 keys 42.6 /
+// 28.8 / 21.2 / 18.8 / 18.9, with a window of 512 after 8000 keys 20.0 / 18.3 /
+// 17.2 / 15.9 / 17.8; 32 / 4 heads x 128 there 11.6 / 11.9 / 11.7 / 12.0 / 15.8
+// and over 1017 keys 14.9 / 13.2 / 12.1 / 12.6 / 16.2.
 template <int D>
 int launch_mq32(const MqArgs &a0, hipStream_t st) {
     MqArgs a = a0;
     const int64_t base = (int64_t)((a.query_len + 31) / 32) * a.num_heads;
     DOE_REQUIRE(base <= 0x7fffffff, DOE_E_UNSUPPORTED, "too many queries");
     a.splits = 1;
-    if (!a.kv_len_dev && base < g_mq_cus) {
-        const int64_t nkb = ((int64_t)min(a.seq_len, a.capacity) + 31) / 32;
-        const int64_t sp = std::min({(int64_t)g_mq_cus / base, nkb / 8, (int64_t)16});
+    if (g_mq_splits > 0) {
+        a.splits = g_mq_splits;
+    } else if (!a.kv_len_dev && base < g_mq_cus) {
+        int64_t keys = std::min(a.seq_len, a.capacity);
+        if (a.causal) keys = std::max<int64_t>(0, std::min(keys, (int64_t)a.start_pos + a.query_len - a.kv_start));
+        int64_t nkb = (keys + 31) / 32;
+        // (32 queries' windows: window + 31 keys, from any place in a block on)
+        if (a.causal && a.window > 0) nkb = std::min(nkb, ((int64_t)a.window + 61) / 32 + 1);
+        const int64_t each = D == 256 && nkb >= 16 ? 2 : 8;
+        const int64_t sp = std::min({(int64_t)g_mq_cus / base, nkb / each, (int64_t)16});
         if (sp > 1) a.splits = (int)sp;
     }
     if (a.splits > 1) {
@@ -783,7 +797,7 @@ int launch_mq(const MqArgs &a0, hipStream_t st) {
         g_mq_cus = cus > 0 ? cus : 256;
     }
     if constexpr (D <= 256) {
-        if (g_mq_splits == 0 && (int64_t)a.capacity * a.row_stride * 2 < ((int64_t)1 << 31))
+        if (g_mq_queries == 0 && (int64_t)a.capacity * a.row_stride * 2 < ((int64_t)1 << 31))
             return launch_mq32<D>(a, st);
     }
     const int G = a.num_heads / a.num_kv_heads;
@@ -864,6 +878,12 @@ namespace doe {
 int mq_set_splits(int value) {
     DOE_REQUIRE(value >= 0 && value <= 16, DOE_E_INVALID, "attn_mq.splits is 0..16");
     g_mq_splits = value;
+    return DOE_OK;
+}
+
+int mq_set_queries(int value) {
+    DOE_REQUIRE(value == 0 || value == 16, DOE_E_INVALID, "attn_mq.queries is 0 or 16");
+    g_mq_queries = value;
     return DOE_OK;
 }
 

@@ -37,6 +37,7 @@ int attn_scratch_setup(int device);
 // Tuning hooks of individual kernels (0 = automatic).
 int attn_set_splits(int value);
 int mq_set_splits(int value);
+int mq_set_queries(int value);
 int attn_set_waves(int value);
 int attn_set_combine(int value);
 int gemm_set_f16_operands(int value);

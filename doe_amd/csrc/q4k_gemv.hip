@@ -1756,6 +1756,8 @@ int doe_tune_set(const char *key, int value) {
         return doe::int4_set_xcd(value);
     } else if (!strcmp(key, "attn_mq.splits")) {
         return doe::mq_set_splits(value);
+    } else if (!strcmp(key, "attn_mq.queries")) {
+        return doe::mq_set_queries(value);
     } else if (!strcmp(key, "attn_decode.splits")) {
         return doe::attn_set_splits(value);
     } else if (!strcmp(key, "attn_decode.waves")) {

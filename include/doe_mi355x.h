@@ -420,9 +420,11 @@ int doe_attn_decode_noalloc(const void *q, int q_f16, const uint16_t *k_cache,
  *            scores scaled by scale, softcapped by attn_softcap; a query with
  *            no visible key writes zeros.
  * query_len 1 runs the split-K decode kernel; query_len > 1 an MFMA flash
- * kernel (16 queries x the query heads of one KV head per workgroup, f32 q
- * as f16 hi + lo, P in f16, f32 accumulation).  head_dim 64/128/256/512.
- * q, k and v must be 16-byte aligned. */
+ * kernel (f32 q as f16 hi + lo, f32 accumulation): at head_dim 64/128/256 32
+ * queries of a head per workgroup, P as f16 hi + lo (2-4e-7 from float64); at
+ * head_dim 512 and over caches of 2 GiB and more 16 queries x the query heads
+ * of one KV head, P in one f16 (1.4e-4).  The visible keys' K and V must be
+ * finite.  q, k and v must be 16-byte aligned. */
 typedef struct {
     uint32_t num_heads, num_kv_heads, head_dim, seq_len, query_len;
     float scale;
@@ -671,7 +673,8 @@ int doe_decode_advance(int32_t *state, int32_t *token, int32_t *ids, int64_t max
  * "int4_gemv.xcd" (1: workgroup ids in plain order, not a row block's K
  * ranges grouped on one XCD), "q8_0_gemv.rows" (1, 2 or 4 rows per wave group), "q8_0_gemv.depth" (1 or
  * 2 blocks loaded ahead), "attn_mq.splits" (1..16 key splits of the
- * 16-query form of the multi-query attention, at any head_dim), "attn_decode.splits",
+ * multi-query attention), "attn_mq.queries" (16: its 16-query form, with P in
+ * one f16, at any head_dim), "attn_decode.splits",
  * "attn_decode.waves" (4: narrow workgroups; 8 or 16: the wide short-context
  * workgroup where the head shape allows it), "attn_decode.combine" (1: the
  * block-reduction split combine instead of the one-wave-per-column form),

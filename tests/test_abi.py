@@ -81,6 +81,8 @@ def test_tune_keys_take_their_documented_values():
         "int4_gemv.kernel": ([0, 1, 2], [3]),
         "int4_gemv.depth": ([0, 2, 3], [1, 4]),
         "int4_gemv.xcd": ([0, 1], [2, -1]),
+        "attn_mq.splits": ([0, 1, 16], [-1, 17]),
+        "attn_mq.queries": ([0, 16], [-1, 1, 32]),
     }
     try:
         for key, (good, bad) in cases.items():

@@ -228,3 +228,177 @@ def test_prompt_blocks_against_float64(dev, d, hq, hkv, ql, start, maxs, window,
         want = p @ v[g, :kv].astype(np.float64) / p.sum(1, keepdims=True)
         tol = 2.0 ** -22 * (8 + 1) + 2.0 ** -24 * np.sqrt(kv)
         assert rel_l2(got[:, h], want) <= tol, (h, rel_l2(got[:, h], want))
+
+
+def float64_rows(q, k, v, key_rows, seen, scale, softcap=0.0):
+    """softmax(q k^T) v in float64: q [ql][hq][d], caches [row][hkv][d], logical
+    key p in row key_rows[p], seen [ql][keys]; also the largest |score|."""
+    hq, hkv = q.shape[1], k.shape[1]
+    out, top = np.zeros(q.shape), 0.0
+    any_key = seen.any(1)
+    for h in range(hq):
+        g = h // (hq // hkv)
+        s = q[:, h].astype(np.float64) @ k[key_rows, g].astype(np.float64).T * scale
+        if softcap:
+            s = np.tanh(s / softcap) * softcap
+        top = max(top, np.abs(s[seen]).max(initial=0.0))
+        s = np.where(seen, s, -np.inf)
+        p = np.exp(s - np.where(any_key, s.max(1), 0.0)[:, None])
+        out[:, h] = p @ v[key_rows, g].astype(np.float64) / np.where(any_key, p.sum(1), 1.0)[:, None]
+    return out, top
+
+
+def seen_keys(ql, keys, start, kv_start=0, window=0):
+    pos, key = start + np.arange(ql)[:, None], np.arange(keys)[None, :] + kv_start
+    return (key <= pos) & ((key > pos - window) if window else True)
+
+
+def bound(queries, top, keys):
+    # the 32-query form: Q in two f16 parts and f32 scores (2^-22 and a few
+    # 2^-24 of the largest score), P in two f16 parts, f32 sums; the 16-query
+    # form rounds P to one f16 (2^-11 of each term, at random)
+    return 2.0 ** -22 * (top + 2) + 2.0 ** -24 * np.sqrt(keys) + (2.0 ** -11 if queries == 16 else 0.0)
+
+
+@pytest.fixture
+def mq_form(dev):
+    def choose(splits, queries):
+        ops.tune("attn_mq.splits", splits)
+        ops.tune("attn_mq.queries", queries)
+    yield choose
+    choose(0, 0)
+
+
+@pytest.mark.parametrize("queries", [0, 16])
+@pytest.mark.parametrize("splits", [0, 1, 2, 3, 5, 16])
+@pytest.mark.parametrize("d,hq,hkv,ql,start,window,softcap", [
+    (64, 2, 1, 33, 10, 12, 30.0), (64, 4, 4, 40, 270, 0, 0.0), (128, 4, 2, 70, 300, 100, 0.0),
+    (256, 8, 4, 33, 10, 12, 30.0), (256, 2, 1, 9, 700, 0, 5.0), (256, 4, 1, 64, 500, 260, 0.0)])
+def test_key_splits_of_both_forms_against_float64(mq_form, d, hq, hkv, ql, start, window, softcap, splits, queries):
+    # 1 to 16 key splits, some of them empty, with windows and softcaps
+    rng = np.random.default_rng(d + ql + start)
+    kv = start + ql
+    q = rng.standard_normal((ql, hq, d)).astype(np.float32)
+    k = rng.standard_normal((kv, hkv, d)).astype(np.float16)
+    v = rng.standard_normal((kv, hkv, d)).astype(np.float16)
+    scale = 1.0 / np.sqrt(d)
+    out = DeviceBuffer.empty((ql, hq, d), np.float32)
+    mq_form(splits, queries)
+    ops.attention_prefill_f16kv(up(q), up(k), up(v), out, num_heads=hq, num_kv_heads=hkv, head_dim=d, query_len=ql,
+                                kv_len=kv, kv_stride=kv, start_pos=start, scale=scale, softcap=softcap,
+                                sliding_window=window, kv_layout=1)
+    want, top = float64_rows(q, k, v, np.arange(kv), seen_keys(ql, kv, start, 0, window), scale, softcap)
+    assert rel_l2(out.download(), want) <= bound(queries, top, kv)
+
+
+@pytest.mark.parametrize("splits", [0, 3])
+@pytest.mark.parametrize("layout,page", [(1, 0), (2, 16), (2, 7)])
+@pytest.mark.parametrize("d,hq,hkv,ql,start,kv_start,window", [
+    (64, 4, 2, 45, 200, 0, 130), (64, 2, 2, 2, 37, 3, 33), (128, 4, 1, 33, 90, 5, 64), (128, 2, 1, 100, 0, 0, 70),
+    (256, 8, 4, 31, 300, 0, 257), (256, 2, 1, 65, 63, 11, 40)])
+def test_ring_and_pages_of_several_queries(mq_form, d, hq, hkv, ql, start, kv_start, window, layout, page, splits):
+    # key p in row (kv_start + p) % window of a ring, or through a page table
+    # with the pages in any order; last key blocks partial, by three splits too,
+    # with the key count from the host and from the device
+    rng = np.random.default_rng(d + ql + start + page)
+    L = start + ql - kv_start
+    if layout == 1:
+        cap, rows, extra = window, (kv_start + np.arange(L)) % window, {}
+    else:
+        npg = -(-(kv_start + L) // page) + 2
+        cap, table = npg * page, rng.permutation(npg).astype(np.uint32)
+        at = kv_start + np.arange(L)
+        rows, extra = table[at // page].astype(np.int64) * page + at % page, {"page_table": up(table)}
+    q = rng.standard_normal((ql, hq, d)).astype(np.float32)
+    k = np.full((cap, hkv, d), np.nan, np.float16)  # rows that hold no key
+    v = np.full((cap, hkv, d), np.nan, np.float16)
+    k[rows] = rng.standard_normal((L, hkv, d))
+    v[rows] = rng.standard_normal((L, hkv, d))
+    scale = 1.0 / np.sqrt(d)
+    want, top = float64_rows(q, k, v, rows, seen_keys(ql, L, start, kv_start, window), scale)
+    mq_form(splits, 0)
+    for source in (0, 1):
+        out = DeviceBuffer.empty((ql, hq, d), np.float32)
+        ops.attention_dispatch(up(q), up(k), up(v), out, kv_capacity=cap, kv_layout=layout, page_size=page,
+                               num_heads=hq, num_kv_heads=hkv, head_dim=d, seq_len=L if source == 0 else 0,
+                               kv_len_source=source, kv_len_buffer=up(np.array([L], np.uint32)) if source else None,
+                               query_len=ql, scale=scale, is_causal=1, start_pos=start, kv_start=kv_start,
+                               sliding_window=window, **extra)
+        err = rel_l2(out.download(), want)
+        assert err <= bound(0, top, L), (source, err)
+
+
+def test_a_short_window_is_not_split_by_the_length_of_the_cache(mq_form):
+    # 17 queries see 80 keys (four blocks) of 8000: one split by itself
+    rng = np.random.default_rng(3)
+    hq, hkv, d, ql, start, window = 8, 4, 256, 17, 7983, 64
+    kv = start + ql
+    q = rng.standard_normal((ql, hq, d)).astype(np.float32)
+    k, v = up(rng.standard_normal((kv, hkv, d)).astype(np.float16)), up(rng.standard_normal((kv, hkv, d)).astype(np.float16))
+    got = []
+    for splits in (0, 1, 16):
+        mq_form(splits, 0)
+        out = DeviceBuffer.empty((ql, hq, d), np.float32)
+        ops.attention_prefill_f16kv(up(q), k, v, out, num_heads=hq, num_kv_heads=hkv, head_dim=d, query_len=ql,
+                                    kv_len=kv, kv_stride=kv, start_pos=start, scale=1 / 16, sliding_window=window,
+                                    kv_layout=1)
+        got.append(out.download())
+    assert np.array_equal(got[0], got[1])
+    assert rel_l2(got[2], got[1]) <= 2.0 ** -21
+
+
+@pytest.mark.parametrize("layout,over", [(0, 0), (0, 1), (2, 0)])
+def test_caches_about_two_gib(mq_form, layout, over):
+    # the keys in the last rows of caches just under 2 GiB (the 32-query form,
+    # 32-bit offsets) and just over (the 16-query form): the same bits as over
+    # a cache of these rows alone
+    rng = np.random.default_rng(5)
+    hq, hkv, d, ql, L = 8, 8, 256, 40, 96
+    cap = (1 << 31) // (hkv * d * 2) - (0 if over else 16)
+    q = up(rng.standard_normal((ql, hq, d)).astype(np.float32))
+    k = rng.standard_normal((L, hkv, d)).astype(np.float16)
+    v = rng.standard_normal((L, hkv, d)).astype(np.float16)
+    common = dict(num_heads=hq, num_kv_heads=hkv, head_dim=d, query_len=ql, scale=1 / 16, is_causal=1, seq_len=L)
+    small = DeviceBuffer.empty((ql, hq, d), np.float32)
+    mq_form(1, 16 if over else 0)
+    ops.attention_dispatch(q, up(k), up(v), small, kv_capacity=L, start_pos=L - ql, **common)
+    mq_form(1, 0)
+    row = hkv * d * 2
+    bk, bv = DeviceBuffer(cap * row), DeviceBuffer(cap * row)
+    for buf, rows in ((bk, k), (bv, v)):
+        buf.view((cap - L) * row, L * row).upload(rows)
+    out = DeviceBuffer.empty((ql, hq, d), np.float32)
+    if layout == 2:  # pages of 16 rows, the last six of the cache
+        table = up(np.arange(cap // 16 - L // 16, cap // 16, dtype=np.uint32))
+        ops.attention_dispatch(q, bk, bv, out, kv_capacity=cap, start_pos=L - ql, kv_layout=2, page_size=16,
+                               page_table=table, **common)
+    else:
+        ops.attention_dispatch(q, bk, bv, out, kv_capacity=cap, start_pos=cap - ql, kv_start=cap - L, **common)
+    assert np.array_equal(out.download(), small.download())
+
+
+@pytest.mark.parametrize("d", [64, 128, 256, 512])
+def test_query_rows_keep_to_themselves(dev, d):
+    # a query of NaN, of an infinity, of zeros, of the largest values changes no
+    # other query's bits; zeros see the mean of the values; a NaN query gives NaN
+    # (head_dim 512's kernel: zeros, as for a query without keys)
+    rng = np.random.default_rng(d)
+    hq, hkv, ql = 2, 1, 40
+    q = rng.standard_normal((ql, hq, d)).astype(np.float32)
+    k = rng.standard_normal((ql, hkv, d)).astype(np.float16)
+    v = rng.standard_normal((ql, hkv, d)).astype(np.float16)
+    bad = q.copy()
+    bad[3, 0, 5], bad[9, 1, 0], bad[17], bad[20], bad[35, :, :] = np.nan, np.inf, 0.0, 3e38, 1e-38
+    outs = []
+    for x in (q, bad):
+        out = DeviceBuffer.empty((ql, hq, d), np.float32)
+        ops.attention_prefill_f16kv(up(x), up(k), up(v), out, num_heads=hq, num_kv_heads=hkv, head_dim=d, query_len=ql,
+                                    kv_len=ql, kv_stride=ql, start_pos=0, scale=0.1, kv_layout=1)
+        outs.append(out.download())
+    same = np.ones((ql, hq), bool)
+    same[3, 0] = same[9, 1] = same[17] = same[20] = same[35] = False
+    assert np.array_equal(outs[0][same], outs[1][same])
+    assert np.isnan(outs[1][3, 0]).all() or d == 512
+    mean = np.cumsum(v.astype(np.float64), 0) / np.arange(1, ql + 1)[:, None, None]
+    for i in (17, 35):
+        assert rel_l2(outs[1][i], np.broadcast_to(mean[i], (hq, d))) <= (1e-3 if d == 512 else 1e-6)
