@@ -702,28 +702,31 @@ namespace doe {
 
 // 64- or 128-row tiles and the K splits (each at least 256 elements of K, at
 // most 32: their partials are written and summed once more), by the least of
-//   blocks of 256 K on the busiest CU x us per block + the partials' traffic.
-// A CU takes 3.6 us per block of a 128-row Q4_K tile with one workgroup or two
-// (5.0 Q8_0, and 0.3 of a block to fill the pipeline), 2.1 of a 64-row one (3.3);
-// the summing pass costs 3.5 us and its bytes at 4 TB/s (Q8_0 8: with 4, three
-// splits of 600 x 4096 x 2304, 48.6 us, lost to one, 52.8; so 1000 x 2304 x 9216
-// 146 -> 142 and the norm + GeGLU of 128 x 18432 x 2304 51.4 -> 49.1.  Q4_K at 8
-// would split the latter, 39 -> 43).  Measured (Q4_K, us, with the rule / the other tile height /
-// two workgroups per CU filled with splits): 128 x 18432 x 2304 39 / 40 / 43
-// (128 rows, one split), 128 x 4096 x 2304 20 / 24 / 28 (64 rows, three),
-// 512 x 2304 x 9216 65 / 92 / 75 (128 rows, three), 20 x 18432 x 2304 23.5
-// against 26 unsplit.
+//   blocks of 256 K on the busiest CU x us per block + the partials' cost.
+// A CU takes 3.8 us per block of a 128-row Q4_K tile with one workgroup or two
+// (5.0 Q8_0), 2.2 of a 64-row one (3.2), and 0.35 of a block to fill the
+// pipeline; the summing pass costs 3.5 us and its bytes at 7 TB/s (tens of MB,
+// read back from the last-level cache).  Chosen over every (height, splits) of 16
+// weight shapes x 19 prompt lengths; of the 31 shapes where it decides other than
+// with the partials at 4 TB/s for Q4_K and 8 for Q8_0 and a fill for Q8_0 alone,
+// 24 are faster (Q4_K 33 x 18432 x 2304 27.6 -> 25.2 us, 400 x 3072 x 3072 38.3 ->
+// 34.9, Q8_0 80 x 1536 x 4096 24.4 -> 21.0, 110 x 2304 x 2048 22.7 -> 19.7), the
+// worst 64 x 9000 x 1152 with GeGLU 17.8 -> 18.9 (200 x 18432 x 2304 Q8_0 with GeGLU
+// over halves, which takes a second pass in any case, 85 -> 92).  Height and splits, us, with
+// the rule / without: Q4_K 128 x 4096 x 2304 64 rows in three 21.6 / unsplit 27;
+// 512 x 2304 x 9216 128 rows in three 66.5 / 64 rows 70.5; Q8_0 128 x 18432 x
+// 2304 128 rows in three 47.2 / unsplit 50.6.
 GemmF32Plan gemm_f32_plan(int64_t m, int64_t n, int64_t k, int fmt, int num_cus) {
     GemmF32Plan p{};
     const int64_t nblk = (padded_k(k, fmt) + 255) / 256;
     double best = 0.0;
     for (int rows = 64; rows <= 128; rows += 64) {
-        const double block_us = rows == 64 ? (fmt == 0 ? 2.1 : 3.3) : (fmt == 0 ? 3.6 : 5.0);
+        const double block_us = rows == 64 ? (fmt == 0 ? 2.2 : 3.2) : (fmt == 0 ? 3.8 : 5.0);
         const int64_t tiles = ((m + rows - 1) / rows) * ((n + 127) / 128);
         for (int64_t want = 1; want <= 32 && want <= nblk && (want == 1 || tiles * want <= 3 * num_cus); ++want) {
             const int64_t per = (nblk + want - 1) / want, splits = (nblk + per - 1) / per;
-            double us = (double)((tiles * splits + num_cus - 1) / num_cus) * ((double)per + (fmt == 0 ? 0.0 : 0.3)) * block_us;
-            if (splits > 1) us += 3.5 + (double)splits * (double)(m * n) * 8e-6 / (fmt == 0 ? 4.0 : 8.0);
+            double us = (double)((tiles * splits + num_cus - 1) / num_cus) * ((double)per + 0.35) * block_us;
+            if (splits > 1) us += 3.5 + (double)splits * (double)(m * n) * 8e-6 / 7.0;
             if (p.tile_rows == 0 || us < best) {
                 best = us;
                 p.tile_rows = rows;
