@@ -240,8 +240,8 @@ __global__ __launch_bounds__(64 * W, 8 / W) void attn_prefill_kernel(PrefillArgs
     // 0: none of them masked, 1: masked, 2: there is none).  At its start K(kb +
     // 1) and V(kb) are in LDS, K(kb + 2) and V(kb + 1) under way; it issues K(kb
     // + 3) and, as V(kb + 1)'s registers come free, V(kb + 2) (past the last: the
-    // last again, never used).  One wave per SIMD: what the vector unit does is
-    // dealt out between the MFMAs, each step its own scheduling region.
+    // last again, never used).  A wave issues in order: what the vector unit does
+    // is dealt out between the MFMAs, each step its own scheduling region.
     uint32_t ks_next = kBlock;  // K(kb + 1)'s place in the ring
     int ks_load = 0;            // K(kb + 3)'s
     auto iter = [&](const int kb, const int mode, float16v &sc, float16v &sn) __attribute__((always_inline)) {
@@ -391,6 +391,8 @@ __global__ __launch_bounds__(64 * W, 8 / W) void attn_prefill_kernel(PrefillArgs
         finish(2);
 }
 
+int g_num_cus = 0;
+
 template <int W>
 int launch(const PrefillArgs &a, int64_t blocks, hipStream_t st) {
     static const hipError_t attr_rc = hipFuncSetAttribute((const void *)attn_prefill_kernel<W>,
@@ -443,11 +445,18 @@ int doe_attn_prefill(const uint16_t *q, const uint16_t *k, const uint16_t *v, vo
     a.pair = (num_heads / num_kv_heads) % 2 == 0;
     a.cols = (int)(a.pair ? num_heads / 2 : num_heads);
     const int64_t rows = a.pair ? 2 * q_len : q_len;  // of a column
+    if (g_num_cus == 0) {
+        int dev = 0, cus = 0;
+        DOE_HIP_CHECK(hipGetDevice(&dev));
+        DOE_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        g_num_cus = cus > 0 ? cus : 256;
+    }
     // Eight waves once the four-wave workgroups (two per CU) come to well over one
-    // round: half of the staging, which then counts (704 of them 30.3 against
-    // 32.7 us, 1024 56 against 60, back to back); up to there four: more, shorter
-    // workgroups (560: 23.1 against 24.6; 512: 36.7 against 39.5; 96: 24 against 33)
-    const bool wide = (rows + 63) / 64 * a.cols > 640;
+    // round, two and a half per CU: half of the staging, which then counts (704 of
+    // them 30.3 against 32.7 us, 1024 56 against 60, back to back); up to there
+    // four: more, shorter workgroups (560: 23.1 against 24.6; 512: 36.7 against
+    // 39.5; 96: 24 against 33)
+    const bool wide = (rows + 63) / 64 * a.cols * 2 > 5 * (int64_t)g_num_cus;
     a.units = (int)(wide ? (rows + 127) / 128 : (rows + 63) / 64);
     a.scale_log2 = scale * 1.4426950408889634f;
     hipStream_t st = (hipStream_t)stream;

@@ -155,8 +155,8 @@ def test_prefill_workgroup_widths(dev, ora, hq, hkv, s, start, causal):
 
 
 def test_prefill_graph_replays(dev):
-    # replays of one captured call (the V^T pre-pass and the attention kernel),
-    # with eager calls in between, all reproduce the eager result exactly
+    # replays of one captured call, with eager calls in between, all reproduce
+    # the eager result exactly
     rng = np.random.default_rng(12)
     hq, hkv, s = 8, 2, 1024
     q = up(to_bf16(rng.standard_normal((s, hq, D), dtype=np.float32)))
@@ -180,6 +180,35 @@ def test_prefill_graph_replays(dev):
         call()
     g.destroy()
     st.destroy()
+
+
+@pytest.mark.parametrize("hq,hkv,s,kv,causal", [(4, 2, 100, 100, True), (3, 3, 70, 200, False)])
+def test_prefill_rows_and_extremes(dev, ora, hq, hkv, s, kv, causal):
+    # values up to the largest bf16 that f16 holds; NaN, infinite and zero
+    # queries change no other query's bits (the heads of a workgroup included)
+    rng = np.random.default_rng(s)
+    q = rng.standard_normal((s, hq, D), dtype=np.float32)
+    k = to_bf16(rng.standard_normal((hkv, kv, D), dtype=np.float32))
+    vf = rng.standard_normal((hkv, kv, D), dtype=np.float32) * 1e4
+    vf[:, ::7, ::3] = 65280.0
+    v = to_bf16(np.clip(vf, -65280.0, 65280.0))
+    start = kv - s if causal else 0
+    got = run(to_bf16(q), k, v, hq, hkv, s, kv, kv, start, 0.1, causal)
+    want = oracle(ora, to_bf16(q), k, v, hq, hkv, s, kv, kv, start, 0.1, causal)
+    assert rel_l2(got, want) <= TOL
+    bad = q.copy()
+    bad[3, 0, 5], bad[40, hq - 1, 0], bad[65] = np.nan, np.inf, 0.0
+    b = to_bf16(np.nan_to_num(bad, nan=1.0, posinf=1.0))
+    b[3, 0, 5], b[40, hq - 1, 0] = 0x7FC0, 0x7F80
+    other = run(b, k, v, hq, hkv, s, kv, kv, start, 0.1, causal)
+    same = np.ones((s, hq), bool)
+    same[3, 0] = same[40, hq - 1] = same[65] = False
+    assert np.array_equal(got[same], other[same])
+    assert np.isnan(other[3, 0]).all()
+    vd = bf16_to_f32(v).astype(np.float64)
+    for h in range(hq):
+        mean = vd[h // (hq // hkv), : start + 66 if causal else kv].mean(0)
+        assert rel_l2(other[65, h], mean) <= TOL
 
 
 def test_prefill_softmax_invariants(dev):
