@@ -189,6 +189,77 @@ def test_gemm_f32_one_sided_rows(dev, ora, m, n, k, minima):
         assert err <= tol, (name, err, tol)
 
 
+@pytest.mark.parametrize("fmt,m,n,k,norm", [
+    ("q4k", 333, 2304, 9216, False), ("q8_0", 333, 2304, 9216, True),  # 128-row tiles, K splits
+    ("q8_0", 300, 1000, 4648, False), ("q8_0", 333, 2304, 1576, True), ("q8_0", 200, 300, 5416, False),  # odd last split
+    ("q4k", 1100, 300, 520, False), ("q8_0", 1100, 300, 520, True), ("q4k", 1290, 1500, 700, True),  # over 8 rows of tiles
+    ("q4k", 70, 200, 5000, True), ("q4k", 70, 200, 5000, False), ("q8_0", 70, 200, 5000, True),
+    ("q4k", 70, 130, 9000, True), ("q8_0", 70, 130, 9000, True), ("q8_0", 70, 130, 9000, False),
+    ("q4k", 40, 130, 13000, True), ("q4k", 40, 130, 13000, False), ("q8_0", 40, 130, 13000, True),
+    ("q8_0", 40, 130, 13000, False)])
+def test_gemm_f32_forms_against_float64(dev, ora, fmt, m, n, k, norm):
+    # tile heights with and without K splits, odd numbers of chunks in the last
+    # split, more than one group of M tiles, and each form of the pre-pass (rows in
+    # registers by width, re-read past 12288 columns) with and without the norm
+    # (which is the rmsnorm op's, bit for bit).  Bound as for one-sided rows; the
+    # Q8_0 blocks are 32 elements, four steps each.
+    from doe_amd import q8_0
+
+    rng = np.random.default_rng(m + n + k)
+    a = (rng.standard_normal((m, k)) * 10.0 ** rng.uniform(-2, 2, (m, 1)) + 0.3).astype(np.float32)
+    w = q4k_with_minima(rng, n, k, "middle") if fmt == "q4k" else q8_0.random_q8_0(rng, n, k)
+    wf = (ora.q4k_dequant_rowwise if fmt == "q4k" else ora.q8_0_dequant)(w, n, k).astype(np.float64)
+    da, x, args = up(a), a, {}
+    if norm:
+        nw = up((0.1 * rng.standard_normal(k)).astype(np.float32))
+        xn = DeviceBuffer.empty((m, k), np.float32)
+        ops.rmsnorm(da, nw, xn, m, k, 1e-6, weight_offset=True)
+        x, args = xn.download(), dict(norm_weight=nw, norm_eps=1e-6, norm_weight_offset=True)
+    out = DeviceBuffer.empty((m, n), np.float32)
+    ops.matmul_gemm_f32_fused(da, up(w), out, m, n, k, fmt, **args)
+    got, want = out.download(), x.astype(np.float64) @ wf.T
+    block, steps = (256, 32) if fmt == "q4k" else (32, 4)
+    tol = 2.0 ** -22 + 2.0 ** -24 * (np.sqrt(steps) + np.sqrt(k / block))
+    worst = max(rel_l2(got[r], want[r]) for r in range(m))
+    print(f"[{fmt} {m}x{n}x{k} norm {norm}] {rel_l2(got, want):.2e}, worst row {worst:.2e} of {tol:.2e}", flush=True)
+    assert worst <= tol
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q8_0"])
+@pytest.mark.parametrize("m,n,k", [(70, 130, 600), (200, 9000, 512)])
+def test_gemm_f32_rows_keep_to_themselves(dev, ora, fmt, m, n, k):
+    # rows at the edges of the f16 scaling (powers of two and just below, the
+    # smallest and largest f32, zeros, one element) hold the bound of any row; a
+    # NaN or infinite row changes no other row's bits
+    from doe_amd import q8_0
+
+    rng = np.random.default_rng(m + k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    peak = np.abs(a).max(1)
+    for r, top in ((1, 1.0), (2, np.nextafter(np.float32(1), np.float32(0))), (5, 65504.0), (33, 2.0 ** 100),
+                   (34, 2.0 ** -100), (40, 2.0 ** 14)):
+        a[r] *= top / peak[r]
+        a[r, 7] = top
+    a[50], a[51] = 0.0, 0.0
+    a[51, 300] = -3.0
+    w = q4k_with_minima(rng, n, k, "middle") if fmt == "q4k" else q8_0.random_q8_0(rng, n, k)
+    wf = (ora.q4k_dequant_rowwise if fmt == "q4k" else ora.q8_0_dequant)(w, n, k).astype(np.float64)
+    dw = up(w)
+    out = DeviceBuffer.empty((m, n), np.float32)
+    ops.matmul_gemm_f32_fused(up(a), dw, out, m, n, k, fmt)
+    got, want = out.download(), a.astype(np.float64) @ wf.T
+    tol = 2.0 ** -22 + 2.0 ** -24 * (np.sqrt(32) + np.sqrt(k / 32))
+    for r in range(m):
+        assert r == 50 and not got[r].any() or rel_l2(got[r], want[r]) <= tol, r
+    bad = a.copy()
+    bad[3, 11], bad[36, 0], bad[60] = np.nan, -np.inf, 3.4e38
+    ops.matmul_gemm_f32_fused(up(bad), dw, out, m, n, k, fmt)
+    rest = np.setdiff1d(np.arange(m), (3, 36, 60))
+    other = out.download()
+    assert np.array_equal(other[rest], got[rest])
+    assert not np.isfinite(other[3]).any() and not np.isfinite(other[36]).any()
+
+
 def test_gemm_prefill_config_sampled(dev, ora):
     # the 31B-class prefill shape: M=2048 tokens, K=5376, N=21504; the oracle
     # evaluates 2048 sampled entries (every row once, at a random column)
