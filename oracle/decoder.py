@@ -163,10 +163,10 @@ class OracleDecoder:
         """One decode step.  Models of the batched prompt's precision (for a
         prompt of at most 32 tokens, one key block of its attention):
         `f16_probs` rounds the attention probabilities to f16 as the prompt's
-        attention does (its f32-accurate GEMMs need no model);
-        `f16_operands` also rounds the layer projections' operands to f16, as
-        the prompt GEMMs' f16-operand form does.  The lm_head and
-        per-layer-embedding GEMVs stay f32."""
+        attention does at head_dim 512 (up to 256 it is f32-accurate, as the
+        GEMMs are, and needs no model); `f16_operands` also rounds the layer
+        projections' operands to f16, as the prompt GEMMs' f16-operand form
+        does.  The lm_head and per-layer-embedding GEMVs stay f32."""
         self.f16_operands = f16_operands
         self.f16_probs = f16_probs or f16_operands
         try:

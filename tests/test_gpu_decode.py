@@ -537,22 +537,15 @@ def test_gemma4_31b_af16_prefill_matches_oracle_decoder(dev, ora):
     assert max(errs) <= 1e-3
 
 
-def _prefill_then_decode(dec, oracle, prompt, n_after, s, f16_prompt=False):
+def _prefill_then_decode(dec, oracle, prompt, n_after, s):
     """Batched prompt, then decode steps; every logits vector against the
-    oracle decoder stepping through the same tokens.  Returns the errors.
-    With `f16_prompt` the oracle's prompt steps round the attention
-    probabilities to f16 as the prompt's attention does, and the first error
-    against the plain f32 oracle is appended last."""
+    f32 oracle decoder stepping through the same tokens.  Returns the errors."""
     dec.prefill(prompt, s)
     s.synchronize()
     got = dec.logits.download()
-    exact = None
-    if f16_prompt:
-        for pos, t in enumerate(prompt):
-            exact = oracle.step(pos, int(t))
     want = None
-    for pos, t in enumerate(prompt):  # rewrites the oracle's cache rows 0..P-1
-        want = oracle.step(pos, int(t), f16_probs=f16_prompt)
+    for pos, t in enumerate(prompt):
+        want = oracle.step(pos, int(t))
     errs = [rel_l2(got, want)]
     tok = int(dec.token.download()[0])
     assert tok == int(np.argmax(want))
@@ -567,8 +560,6 @@ def _prefill_then_decode(dec, oracle, prompt, n_after, s, f16_prompt=False):
         tok = int(dec.token.download()[0])
         assert tok == int(np.argmax(want)), pos
         ids.append(tok)
-    if f16_prompt:
-        errs.append(rel_l2(got, exact))
     return errs
 
 
@@ -590,26 +581,23 @@ def test_prefill_matches_oracle_decoder(dev, ora):
     assert max(errs) <= 1e-3
 
 
-# The batched prompt's GEMMs run f32-accurate (activation and dequantised
-# weight each carried as an f16 hi + lo pair, the product at f32-GEMV
-# accuracy, test_gpu_gemm.py); its attention rounds the probabilities to f16.
-# In the random Q8_0 model (keys of ~7) attention is soft and the layers are
-# badly conditioned: its decode steps, f32 throughout, already sit 3e-4 from
-# the float64 oracle at 26 layers (test_full_size_first_steps), and the
-# prompt's f16 probabilities reach the logits through every later layer.
-# With f16-operand GEMMs (one rounding per operand) the 26-layer prompt
-# logits sat 1.2e-2 from the f32 oracle; f32-accurate, 6.6e-4.  So these
-# tests check layer 0's cache rows -- the Q8_0 GEMM, the rotate-half RoPE and
-# the cache write, before any amplification -- against the f32 oracle, and
-# the prompt logits and the decode steps after it within 1e-3 of both the
-# oracle that rounds the prompt's probabilities the same way and the plain
-# f32 oracle.
+# The batched prompt's GEMMs run f32-accurate (activation as f16 hi + lo, the
+# weights as their integers, test_gpu_gemm.py), and so does its attention up to
+# head_dim 256 (Q and the probabilities as f16 hi + lo).  In the random Q8_0
+# model (keys of ~7) attention is soft and the layers are badly conditioned: its
+# decode steps, f32 throughout, already sit 3e-4 from the float64 oracle at 26
+# layers (test_full_size_first_steps).  So these tests check layer 0's cache
+# rows -- the Q8_0 GEMM, the rotate-half RoPE and the cache write, before any
+# amplification -- and the logits of the prompt and of the decode steps after
+# it, against the f32 oracle within 1e-3: the prompt 2.2e-5 and 5.5e-4 at 2 and
+# 26 layers, the steps (each rounding one more K/V row to f16) up to 1.9e-4 and
+# 5.5e-4; 1.2e-2 at 26 layers with f16-operand GEMMs.  Probabilities rounded to
+# f16 put the 2-layer prompt 1.3e-4 away, so that one is held to 1e-4.
 # (layer 0's K/V rows are f16 in the cache: an f32 value ~1e-7 away from the
-# oracle's can round to the neighbouring f16, 2^-11 apart; 2.2e-5 measured at
-# 2 layers)
+# oracle's can round to the neighbouring f16, 2^-11 apart; 9.7e-6 and 3.3e-5
+# measured)
 Q8_PREFILL_KV0 = {2: 1e-4, 26: 1e-4}
 Q8_PREFILL_TOL = {2: 1e-3, 26: 1e-3}
-Q8_PREFILL_DRIFT = {2: 1e-3, 26: 1e-3}
 
 
 def _layer0_cache_err(dec, oracle, P):
@@ -631,13 +619,13 @@ def test_prefill_q8_0_matches_oracle_decoder(dev, ora):
     s = Stream()
     oracle = OracleDecoder(dec)
     prompt = np.array([3, 900, 4001, 17, 17, 256, 1024, 5, 77, 3000, 12, 1, 2, 3], np.int32)
-    *errs, drift = _prefill_then_decode(dec, oracle, prompt, 4, s, f16_prompt=True)
+    errs = _prefill_then_decode(dec, oracle, prompt, 4, s)
     kv0 = _layer0_cache_err(dec, oracle, prompt.size)
-    print(f"[prefill q8_0 small] layer-0 K/V rows {kv0:.1e}, logits rel_l2 {['%.1e' % e for e in errs]}, "
-          f"f32 oracle {drift:.1e}", flush=True)
+    print(f"[prefill q8_0 small] layer-0 K/V rows {kv0:.1e}, logits rel_l2 {['%.1e' % e for e in errs]}",
+          flush=True)
     assert kv0 <= Q8_PREFILL_KV0[2]
+    assert errs[0] <= 1e-4  # the prompt's own logits
     assert max(errs) <= Q8_PREFILL_TOL[2]
-    assert drift <= Q8_PREFILL_DRIFT[2]
 
 
 def test_prefill_full_size(dev, ora):
@@ -674,7 +662,7 @@ def test_prefill_q4k_soft_attention(dev, ora):
     s = Stream()
     oracle = OracleDecoder(dec)
     prompt = np.array([12345, 200000, 7, 7, 99999, 1, 250000, 31337, 42, 100, 65535, 3], np.int32)
-    *errs, drift = _prefill_then_decode(dec, oracle, prompt, 3, s, f16_prompt=True)
+    errs = _prefill_then_decode(dec, oracle, prompt, 3, s)
     # the prompt's attention is soft: layer 0, head 0, last prompt query
     P, c, L0 = prompt.size, cfg, oracle.layers[0]
     x = ora.embed_gather(oracle.embed, prompt[-1:], c.embed_scale)[0]
@@ -682,10 +670,9 @@ def test_prefill_q4k_soft_attention(dev, ora):
     q = ora.rope(qkv[: L0["q_dim"] + L0["kv_dim"]], L0["table"], 1, c.heads + c.kv_heads, c.head_dim, P - 1)[:c.head_dim]
     sc = np.asarray(L0["kc"][0, :P], np.float64) @ q / np.sqrt(c.head_dim)
     pmax = float(np.exp(sc - sc.max()).max() / np.exp(sc - sc.max()).sum())
-    print(f"[prefill q4k soft] logits rel_l2 {['%.1e' % e for e in errs]}, f32 oracle {drift:.1e}, "
+    print(f"[prefill q4k soft] logits rel_l2 {['%.1e' % e for e in errs]}, "
           f"layer-0 head-0 max probability {pmax:.2f}", flush=True)
     assert max(errs) <= 1e-3
-    assert drift <= 1e-3
     assert pmax < 0.9
 
 
@@ -789,10 +776,9 @@ def test_prefill_q8_0_full_size(dev, ora):
     s = Stream()
     oracle = OracleDecoder(dec)
     prompt = np.array([12345, 200000, 7, 99999, 250000, 3], np.int32)
-    *errs, drift = _prefill_then_decode(dec, oracle, prompt, 1, s, f16_prompt=True)
+    errs = _prefill_then_decode(dec, oracle, prompt, 1, s)
     kv0 = _layer0_cache_err(dec, oracle, prompt.size)
-    print(f"[prefill 2B q8_0] layer-0 K/V rows {kv0:.1e}, logits rel_l2 {['%.1e' % e for e in errs]}, "
-          f"f32 oracle {drift:.1e}", flush=True)
+    print(f"[prefill 2B q8_0] layer-0 K/V rows {kv0:.1e}, logits rel_l2 {['%.1e' % e for e in errs]}",
+          flush=True)
     assert kv0 <= Q8_PREFILL_KV0[26]
     assert max(errs) <= Q8_PREFILL_TOL[26]
-    assert drift <= Q8_PREFILL_DRIFT[26]

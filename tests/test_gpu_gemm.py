@@ -53,8 +53,8 @@ def test_gemm_matches_oracle(dev, ora, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(128, 2304, 9216), (128, 4096, 2304), (17, 300, 2048), (128, 18432, 2304),
                                    (3, 64, 1024)])
 def test_gemm_f32_prompt_shapes(dev, ora, m, n, k):
-    # the decoder's batched prompt: f32 activations, few 128 x 128 tiles, so K
-    # runs split over the grid (partial tiles summed in split order); float64
+    # the decoder's batched prompt: f32 activations, few tiles, so K runs split
+    # over the grid (partial tiles summed in split order); float64
     # reference over the dequantised weights.  The f32-accurate kernel (hi +
     # lo operands) sits at f32-GEMV accuracy; the f16-operand form (tuned) at
     # one f16 rounding per operand, inside the 1e-3 contract.
@@ -86,8 +86,9 @@ def test_gemm_f32_prompt_shapes(dev, ora, m, n, k):
                                    (130, 257, 2304), (1, 3, 32)])
 def test_q8_0_gemm_f32(dev, ora, m, n, k):
     # Q8_0 rows (34-byte blocks, 2-byte aligned; a K that is no multiple of 32
-    # zero-pads the last block) through the 128 x 128 kernel with its K split;
-    # float64 reference over the oracle's dequantised rows
+    # zero-pads the last block) through the f32-accurate kernel and, tuned, the
+    # 128 x 128 f16-operand one, both with their K splits; float64 reference over
+    # the oracle's dequantised rows
     from doe_amd import q8_0
 
     rng = np.random.default_rng(m * 3 + n + k)
@@ -120,8 +121,9 @@ def test_gemm_f32_tile_edges(dev, ora, fmt, m, n, k):
     # around the edges of the 32-row fragments, the 64 / 128 x 128 tiles and
     # the 32 / 64 / 256 pieces of K, without and with K splits, plain, with the
     # residual and with GeGLU of column pairs.  Bound: A's two f16 parts carry
-    # it to 2^-22, f32 sums of k terms to 2^-24 sqrt(k), the minima's sums
-    # cancel against the scales' (a factor of 2).
+    # it to 2^-22, f32 sums of k terms to 2^-24 sqrt(k); twice that, for a
+    # Q4_K block's sum of integers and its remainders' sum, each as large as a
+    # term of the result.
     from doe_amd import q8_0
 
     rng = np.random.default_rng(m + 3 * n + k)
