@@ -13,11 +13,12 @@
 // tanh(s / cap) * cap, softmax over the visible keys; a query without keys
 // writes zeros.
 //
-// Kernels.  head_dim 64 / 128 / 256 runs attn_mq32_kernel (below); head_dim 512
-// (whose Q and O do not fit one wave's registers there) and caches of 2 GiB and
-// more (and attn_mq.queries = 16) attn_mq_kernel: one workgroup = 16
-// consecutive queries x HG query heads of one KV head (one wave per head), keys in blocks of 32 staged in LDS and shared by
-// the waves: K row-major for S = Q K^T and V transposed for O = P V, both on
+// Kernels.  head_dim 64 / 128 / 256 runs attn_mq32_kernel (below).  head_dim 512
+// (whose Q and O do not fit one wave's registers there), caches of 2 GiB and
+// more and attn_mq.queries = 16 run attn_mq_kernel: one workgroup = 16
+// consecutive queries x HG query heads of one KV head (one wave per head), keys
+// in blocks of 32 staged in LDS and shared by the waves: K row-major for S = Q
+// K^T and V transposed for O = P V, both on
 // v_mfma_f32_16x16x32_f16.  Q is f32: each query row is scaled by a power of
 // two (max near 2^14) and split into f16 hi + lo (~22 bits), so the scores
 // carry f32 quality; P is rounded to f16 once (used for both the numerator
@@ -347,9 +348,9 @@ __global__ __launch_bounds__(NTH) void attn_mq_kernel(MqArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// head_dim 64 / 128 / 256: one workgroup = 32 queries of one
-// head; its four waves take every fourth block of 32 keys and merge their (o,
-// m, l) in LDS at the end, so no wave waits for another in between.
+// head_dim 64 / 128 / 256: one workgroup = 32 queries of one head; its four waves
+// take every fourth block of 32 keys and merge their (o, m, l) in LDS at the end,
+// so no wave waits for another in between.
 //   * S^T = K Q^T on v_mfma_f32_32x32x16_f16: a query per lane column (its max
 //     and sum are one lane-half exchange), Q as f16 hi + lo in registers.
 //   * S^T's sums are P^T's operand order of O^T = V^T P^T as they stand (the
@@ -370,8 +371,8 @@ __global__ __launch_bounds__(NTH) void attn_mq_kernel(MqArgs a) {
 // for a short prompt by the 4 us of launch, Q and first K before it.  us, with
 // the 16-query kernel above (32-key blocks behind two barriers, V transposed
 // by 2-byte stores) in brackets: 1000 tokens, 8 / 4 heads x 256 28 (80); 128
-// tokens 11 (18); 1000 tokens, 16 / 4 x 128 20.5 (60.6); 1500 tokens, 16 / 4 x
-// 64 18.9 (84); 40 queries over 8000 keys 31 (70).
+// tokens 11 (18); 1000 tokens, 16 / 4 x 128 19-20.5 (60.6); 1500 tokens, 16 / 4 x
+// 64 17.5-18.9 (84); 40 queries, 8 / 4 x 256, over 8000 keys 30 (70).
 // ---------------------------------------------------------------------------
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));

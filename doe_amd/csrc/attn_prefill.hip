@@ -36,9 +36,9 @@
 // unit about 1300); otherwise the workgroup with the most key blocks.  us, with
 // 128 queries of one head per workgroup, every wave reading all keys (32 KB of
 // LDS per 32 MFMAs, the LDS port's own rate) and V^T from a pre-pass, in
-// brackets: 2048 x 32 / 16 heads 47.8 (54.6); 2048 x 8 / 8 26.8 (44.6); 1500
-// after 512 x 4 / 4 24.3 (43.0); 1100 x 32 / 16 23.1 (34.8); 65 x 4 / 4 6.2
-// (10.6).  Two tiles of 32 rows to a wave (half of the LDS reads, one wave per
+// brackets, timed in turn: 2048 x 32 / 16 heads 48.6-49.6 (54.6-55.8; alone under
+// sustained load 54-56); 2048 x 8 / 8 27-28 (44.6); 1500 after 512 x 4 / 4 24.5
+// (43.0); 1100 x 32 / 16 22.9 (34.8); 65 x 4 / 4 6.0 (10.6).  Two tiles of 32 rows to a wave (half of the LDS reads, one wave per
 // SIMD) took 55 and 43 on the first two; three blocks of K in flight instead of
 // two, or a block's first K operands read before the barrier, changed nothing.
 #include "common.h"

@@ -36,10 +36,10 @@
 // MFMAs (512 cycles), 16 fragment reads and ~25 VALU operations.
 // Measured (us per call, pre-pass and second pass included; the three-product
 // kernel with per-workgroup dequantisation that this replaced in brackets):
-// Q4_K GeGLU 1000 x 18432 x 2304 188 (391: bound by the matrix cores, the
-// clock down to 1.8 GHz under them), Q8_0 333 x 2304 x 9216 58-62 (83);
-// 128-token calls are bound by the one or two waves per SIMD
-// that a short prompt gives.
+// Q4_K GeGLU 1000 x 18432 x 2304 189 (391-398; matrix cores busy 56 % of the
+// kernel's cycles, the clock down to 1.7 GHz under them), Q8_0 333 x 2304 x 9216
+// 61-63 (83); 128-token calls are bound by the one or two waves per SIMD that a
+// short prompt gives.
 #include "gemm_f32.h"
 
 #include <math.h>

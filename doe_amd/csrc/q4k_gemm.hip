@@ -19,8 +19,10 @@
 //     packed fma.  The relative error of w is ~2^-11, far inside the rel-L2
 //     1e-3 contract; a bf16 B (8 bits) would sit at ~1.1e-3.
 //
-// doe_q8_0_gemm_f32 runs the 128 x 128 kernel over Q8_0 rows (34-byte blocks
-// of an f16 scale and 32 int8 quants), dequantised to f16 the same way.
+// f32 activations (doe_q4k_gemm_f32, doe_q8_0_gemm_f32 and the fused form) run
+// gemm_f32.hip; under quant_gemm.f16_operands they run the kernels here, rounded
+// once to f16, Q8_0 rows (34-byte blocks of an f16 scale and 32 int8 quants) on
+// the 128 x 128 kernel, dequantised to f16 the same way.
 //
 // Tiling: problems with at least 256 tiles of 256 x 256 use q4k_gemm_pipe_kernel
 // (four waves side by side in N, raw B blocks in LDS dequantised per wave,
@@ -127,10 +129,9 @@ __global__ __launch_bounds__(256) void a_rows_to_f16_kernel(const uint16_t *__re
     }
 }
 
-// The same pre-pass for f32 A: each row scaled by 2^sig[m] (max|A[m]| just
-// under 2^14) and rounded once to f16 (11 significant bits).
-// f32 rows to f16 with a per-row power-of-two scale (as a_rows_to_f16_kernel
-// for bf16), optionally through RMSNorm first (the input_norm /
+// The same pre-pass for f32 A, f16 operands: each row scaled by 2^sig[m]
+// (max|A[m]| just under 2^14) and rounded once to f16 (11 significant bits),
+// optionally through RMSNorm first (the input_norm /
 // post_attn_norm step folded into the projection that consumes it; the
 // normalised values are those of the rmsnorm op bit for bit: the same
 // per-thread f32 sums of squares over k = t, t + 256, ..., the same
@@ -739,10 +740,9 @@ __global__ __launch_bounds__(256) void q4k_gemm_pipe_kernel(GemmArgs g) {
     }
 }
 
-// c = sum of the K splits' partial tiles (split order, so the result is
-// the same on every run).
-// c = the split sum (+ res: the attn_residual / ffn_residual step, c may
-// be res), the splits added in order, then the residual.
+// c = the sum of the K splits' partial tiles (+ res: the attn_residual /
+// ffn_residual step, c may be res), the splits added in order (the same result
+// on every run), then the residual.
 __global__ __launch_bounds__(256) void sum_splits_kernel(const float *__restrict__ part, float *c, size_t mn,
                                                          int splits, const float *res) {
     const size_t n4 = mn / 4;
@@ -787,7 +787,8 @@ __global__ __launch_bounds__(256) void sum_splits_geglu_kernel(const float *__re
     }
 }
 
-// Library-owned workspace (grow-only) for the f16 copy of A and its row scales.
+// Library-owned workspace (grow-only): the f16 copy of A with its row scales (and
+// sub-block sums), and the K splits' partial tiles.
 std::mutex g_ws_mu;
 void *g_ws = nullptr;
 size_t g_ws_bytes = 0;
@@ -825,7 +826,7 @@ int sum_parts(const float *part, float *c, int64_t m, int64_t n, int splits, con
     return DOE_OK;
 }
 
-// fmt 0: B Q4_K_M rows; fmt 1: B Q8_0 rows (small-tile kernel only)
+// fmt 0: B Q4_K_M rows; fmt 1: B Q8_0 rows (f32 activations only)
 int gemm_impl(const void *a, bool a_f32, const void *b_q4k, float *c, int64_t m, int64_t n, int64_t k,
               doe_stream_t stream, int fmt = 0, const GemmFusion &fu = GemmFusion()) {
     const uint16_t *a_bf16 = a_f32 ? nullptr : (const uint16_t *)a;
@@ -958,10 +959,6 @@ int gemm_impl(const void *a, bool a_f32, const void *b_q4k, float *c, int64_t m,
 }
 
 }  // namespace
-
-extern "C" {
-
-}  // extern "C"
 
 namespace doe {
 int gemm_set_f16_operands(int v) {

@@ -600,8 +600,8 @@ class Decoder:
         input_norm + q/k/v_proj as one M-row GEMM, rope_q / rope_k with the
         cache write, causal attention of the whole prompt, o_proj +
         attn_residual, post_attn_norm + gate/up_proj + activation, down_proj +
-        ffn_residual -- each "+" folded into the GEMM's pre-pass or the pass
-        that sums its K splits), then the last token's final norm + lm_head +
+        ffn_residual -- each "+" folded into the GEMM's pre-pass, its epilogue or
+        the pass that sums its K splits), then the last token's final norm + lm_head +
         sample.
         Q4_K layers run the Q4_K GEMM, Q8_0 layers the Q8_0 GEMM; both the
         interleaved-pair RoPE of their decode step.

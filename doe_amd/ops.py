@@ -66,8 +66,8 @@ def matmul_q4k_gemm(a_bf16: DeviceBuffer, weight: DeviceBuffer, output: DeviceBu
 
 def matmul_q4k_gemm_f32(a: DeviceBuffer, weight: DeviceBuffer, output: DeviceBuffer, m: int, n: int, k: int,
                         stream=None) -> None:
-    """``matmul_q4k`` at M > 1 with f32 activations a [m][k] (rounded to f16
-    per row by the GEMM's pre-pass): output f32 [m][n]."""
+    """``matmul_q4k`` at M > 1 with f32 activations a [m][k], f32-accurate
+    (carried as f16 hi + lo): output f32 [m][n]."""
     _q4k_weight_check(weight, n, k)
     _need(a, m * k * 4, "a")
     _need(output, m * n * 4, "output")
@@ -126,7 +126,7 @@ def geglu_halves(gate_up: DeviceBuffer, output: DeviceBuffer, rows: int, n: int,
 def matmul_q8_0_gemm_f32(a: DeviceBuffer, weight: DeviceBuffer, output: DeviceBuffer, m: int, n: int, k: int,
                          stream=None) -> None:
     """``matmul`` with quantFormat ``q8_0`` at M > 1: output f32 [m][n] =
-    a f32 [m][k] @ dequant(weight)[n][k]^T (weights rounded to f16 once)."""
+    a f32 [m][k] @ dequant(weight)[n][k]^T, f32-accurate."""
     _need(weight, n * _q8_0.row_bytes(k), "weight")
     _need(a, m * k * 4, "a")
     _need(output, m * n * 4, "output")

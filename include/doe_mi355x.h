@@ -268,7 +268,7 @@ int doe_q8_0_gemm_f32(const float *a, const void *b_q8_0, float *c, int64_t m, i
 /* doe_q4k_gemm_f32 (weight_format 0) or doe_q8_0_gemm_f32 (1) with the
  * prefill steps around a projection folded in (gemma-3-270m-smoke.json:
  * 10-25): input_norm / post_attn_norm (norm_weight non-NULL: a's rows go
- * through RMSNorm, bit for bit the doe_rmsnorm op, before the f16 pre-pass),
+ * through RMSNorm, bit for bit the doe_rmsnorm op, as the pre-pass reads them),
  * attn_residual / ffn_residual (residual non-NULL: c = a W^T + residual,
  * residual may be c), or the GeGLU activation over the gate/up projection
  * (activation 1: columns (2j, 2j + 1) as doe_geglu_pairs; 2: columns (j, j +
