@@ -15,11 +15,12 @@
 //     result's own terms.  (With b = sc q and the minima in the second sum the
 //     two cancel wherever the activations of a row have a common sign.)
 //   * Q8_0: b = q (int8); a 32-element block's sum is d sum(q x).
-// Measured, rows of A with mean 0 to 30 deviations or after ReLU, K 2304 to
-// 13000: Q4_K 1.3-1.8e-7 from float64, Q8_0 1.0-1.4e-7.  (Splitting the
-// dequantised f32 weight into f16 hi + lo instead takes a third product per
-// step and ~6 VALU operations per weight instead of 1.1, and gives 1.9-2.6e-7;
-// b = sc q takes 4 % less time here, and gives 3.2e-7, with a mean 1.4-2.9e-6.)
+// Measured, rows of A with mean 0 to 30 deviations or after ReLU, minima tied to
+// the scales or not, K 2304 to 13000: Q4_K 1.3-1.8e-7 from float64, Q8_0
+// 1.1-1.7e-7.  (Splitting the dequantised f32 weight into f16 hi + lo instead
+// takes a third product per step and ~6 VALU operations per weight instead of
+// 1.1, and gives 1.9-3.7e-7; b = sc q takes 4 % less time here, and gives
+// 3.2e-7, with a mean 1.4-3.0e-6.)
 //
 // Layout.  The pre-pass writes A in operand order: per 32 rows and 32
 // elements of K four 1 KB fragments (step 0 hi, lo, step 1 hi, lo), each the
